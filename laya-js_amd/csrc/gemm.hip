@@ -40,6 +40,12 @@ namespace hb {
 
 const float* rope_table(uintptr_t ctx, int64_t L, int64_t D, double base);
 
+// gemm_f32.hip: f32 linear layers on the matrix cores
+bool f32_linear_ok(uintptr_t x, int64_t ldx, uintptr_t w, int64_t K, int bits, int group);
+void f32_linear(hipStream_t st, int cus, const float* x, int64_t ldx, const float* w, const uint8_t* q, const uint16_t* scales,
+                const uint16_t* zeros, int bits, int group, int aff, const float* bias, const float* r, int64_t ldr,
+                float* y, int64_t ldy, int M, int N, int K, bool geglu);
+
 // ------------------------------------------------------------------ SIMT kernel (f32 path, fallback)
 
 struct QWs {  // quantized weight for the SIMT kernel (bits = 0: plain)
@@ -220,6 +226,9 @@ extern "C" int hb_linear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintpt
     if (dot_shape(M, N, K)) {
       gemm_dot<<<(unsigned)((M * N + 3) / 4), 256, 0, st>>>(dt, (const void*)x, ldx, (const void*)w, qw, b, r, ldr,
                                                            (void*)y, ldy, (int)M, (int)N, (int)K, geglu ? 1 : 0);
+    } else if (dt == HB_F32 && f32_linear_ok(x, ldx, w, K, 0, 1)) {
+      f32_linear(st, cu_count(ctx), (const float*)x, ldx, (const float*)w, nullptr, nullptr, nullptr, 0, 1, 0, (const float*)b,
+                 (const float*)r, ldr, (float*)y, ldy, (int)M, (int)N, (int)K, geglu);
     } else {
       gemm_simt<<<grid, 256, 0, st>>>(dt, (const void*)x, ldx, (const void*)w, qw, b, r, ldr, (void*)y, ldy, (int)M,
                                       (int)N, (int)K, geglu ? 1 : 0);
@@ -357,6 +366,10 @@ extern "C" int hb_qlinear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintp
     if (dot_shape(M, N, K)) {
       gemm_dot<<<(unsigned)((M * N + 3) / 4), 256, 0, st>>>(dt, (const void*)x, ldx, nullptr, q, b, r, ldr, (void*)y,
                                                            ldy, (int)M, (int)N, (int)K, geglu ? 1 : 0);
+    } else if (dt == HB_F32 && f32_linear_ok(x, ldx, qw, K, bits, group) && scales % 2 == 0 && zeros % 2 == 0) {
+      f32_linear(st, cu_count(ctx), (const float*)x, ldx, nullptr, (const uint8_t*)qw, (const uint16_t*)scales,
+                 (const uint16_t*)zeros, bits, group, mode, (const float*)b, (const float*)r, ldr, (float*)y, ldy,
+                 (int)M, (int)N, (int)K, geglu);
     } else {
       gemm_simt<<<grid, 256, 0, st>>>(dt, (const void*)x, ldx, nullptr, q, b, r, ldr, (void*)y, ldy, (int)M, (int)N,
                                       (int)K, geglu ? 1 : 0);
