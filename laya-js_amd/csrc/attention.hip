@@ -20,7 +20,9 @@
 // Backend.rope.  The output is written row-major or, for the attention output
 // projection, in the panel order of the GEMM's X operand.
 //
-// sdpa_simt: the f32 path and the fallback for other head dims / layouts.
+// sdpa_f32_mfma: the f32 path for head dim 64, on v_mfma_f32_32x32x2_f32.
+//
+// sdpa_simt: the fallback for other head dims / layouts.
 //
 // hb_sdpa_noalloc: hb_sdpa without RoPE for callers that cannot allocate; its
 // mask summary goes to `scratch`, a file-scope device array.
@@ -588,6 +590,280 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void s
   }
 }
 
+// ------------------------------------------------------------------ f32 MFMA kernel (D = 64)
+
+// Flash attention in f32 on v_mfma_f32_32x32x2_f32.  A block owns 32 queries
+// of one (b, h); its four waves take the 32-key tiles those queries can see in
+// turn, each with its own running max, sum and output, and merge them in LDS
+// at the end, so a short sequence still runs its key tiles side by side and no
+// wave waits for another in between.  What bounds it is the f32 matrix rate:
+// a tile is 64 MFMAs of 64 cycles against 16 KB of K and V, so K goes through
+// a wave-private LDS tile (rotated by RoPE on the way when fused) and V
+// straight into operand registers, a whole 128-byte line per 32 lanes.
+// S^T = K . Q^T leaves lane l with the scores of query l % 32 for keys
+// 8 * (r / 4) + 4 * (l / 32) + r % 4, which are the columns the B operand of
+// O^T += V^T . P^T takes when MFMA step r multiplies keys 8 * (r / 4) + r % 4
+// and + 4: P stays in registers.
+// Scores, probabilities and sums are f32; exp is the library's expf.
+// Measured (12 heads): B = 8, T = 512, padded, sliding window 5820 -> 96 us
+// (sdpa_simt before, one query per wave and every key rotated per query),
+// B = 1, T = 93 104 -> 12 us, B = 1, T = 8192 without a window 88 TFLOP/s.
+constexpr int kFQ = 32;  // queries per block
+constexpr int kFK = 32;  // keys per tile
+constexpr int kFW = 4;   // waves per block
+
+__global__ __launch_bounds__(kFW * 64) __attribute__((amdgpu_waves_per_eu(2))) void sdpa_f32_mfma(
+    const float* __restrict__ Q, S4 qs, const float* __restrict__ K, S4 ks, const float* __restrict__ V, S4 vs,
+    const uint8_t* __restrict__ mask, S4 ms, const uint8_t* __restrict__ cls, float* __restrict__ O, S4 os, int Lq,
+    int Lk, float scale, const float2* __restrict__ tabq, const float2* __restrict__ tabk, int nqt, int nh) {
+  __shared__ __attribute__((aligned(16))) float buf[kFW][kFK * 64];  // K tiles; the partial outputs at the end
+  __shared__ uint16_t todo[2 * kMaxKeyTiles];  // key tiles to visit: 2 * tile + mixed (Lk < 40960: sdpa_takes_f32)
+  __shared__ int ntodo;
+  __shared__ float part_m[kFW][kFQ], part_l[kFW][kFQ];
+
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lg = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the query tiles of one (b, h) share K and V: consecutive blocks of one XCD
+  const int t = xcd_tile(blockIdx.x, gridDim.x);
+  const int qt = t % nqt, bh = t / nqt, h = bh % nh, b = bh / nh;
+  const int q0 = qt * kFQ, q = q0 + l32;
+  const int nkt = (Lk + kFK - 1) / kFK;
+  const float* Kb = K + b * ks.s[0] + h * ks.s[1];
+  const float* Vb = V + b * vs.s[0] + h * vs.s[1];
+
+  // This lane's query: element e of qf[i] is column 8 * i + 4 * lg + e, the
+  // columns its half supplies to MFMA steps e of chunk pair i
+  float4v qf[8];
+  {
+    const float* qp = Q + b * qs.s[0] + h * qs.s[1] + (int64_t)(q < Lq ? q : Lq - 1) * qs.s[2] + 4 * lg;
+#pragma unroll
+    for (int i = 0; i < 8; i++) qf[i] = *(const float4v*)(qp + 8 * i);
+    if (tabq != nullptr) {
+      const float2* tp = tabq + (int64_t)(q < Lq ? q : Lq - 1) * 32 + 4 * lg;
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float2 cs = tp[8 * i + e];
+          const float x0 = qf[i][e], x1 = qf[i + 4][e];
+          qf[i][e] = fmaf(-x1, cs.y, x0 * cs.x);
+          qf[i + 4][e] = fmaf(x0, cs.y, x1 * cs.x);
+        }
+    }
+  }
+
+  // The key tiles some query of the block sees, in order, from the mask
+  // summary (classes of 16 queries x 64 keys) where there is one; wave 0
+  // packs 64 tiles at a time.
+  if (wave == 0) {
+    int n = 0;
+    for (int base = 0; base < nkt; base += 64) {
+      const int kt = base + lane;
+      int c = 0;  // 0 skip, 1 all visible, 2 mixed
+      if (kt < nkt) {
+        if (mask == nullptr) {
+          c = (kt + 1) * kFK <= Lk ? 1 : 2;
+        } else if (cls == nullptr) {
+          c = 2;
+        } else {
+          const int g = (q0 >> 4) & 7, nkt64 = (Lk + kBK - 1) / kBK, nqt128 = (Lq + kBQ - 1) / kBQ;
+          const uint8_t* p = cls + (((int64_t)b * nqt128 + q0 / kBQ) * nkt64 + (kt >> 1)) * kNW + g;
+          // (a group past Lq has class 0: its queries are not stored)
+          const int c0 = p[0], c1 = q0 + 16 < Lq ? p[1] : p[0];
+          c = c0 == c1 ? c0 : 2;
+        }
+      }
+      const uint64_t m = __ballot(c != 0);
+      if (c != 0) todo[n + __popcll(m & ((1ull << lane) - 1))] = (uint16_t)(2 * kt + (c == 2));
+      n += __popcll(m);
+    }
+    if (lane == 0) ntodo = n;
+  }
+  __syncthreads();
+  const int nt = ntodo;
+
+  // K tile staging: 8 lanes per row; lane c8 of a row holds its chunks c8 and
+  // c8 + 8 (columns 4 * c8 .. and their rotation partners + 32)
+  const int kr = lane >> 3, c8 = lane & 7;
+  float4v klo[4], khi[4];
+  auto load_k = [&](int kt) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int key = kt * kFK + i * 8 + kr;
+      const float* p = Kb + (int64_t)(key < Lk ? key : Lk - 1) * ks.s[2] + 4 * c8;
+      klo[i] = *(const float4v*)p;
+      khi[i] = *(const float4v*)(p + 32);
+    }
+  };
+  // chunk c of row r at c ^ (r & 15): a 16-lane pass of the fragment reads
+  // (16 rows, one chunk) covers all 64 banks
+  auto kslot = [](int r, int c) { return r * 64 + ((c ^ (r & 15)) << 2); };
+  float* kb = buf[wave];
+  auto store_k = [&](int kt) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int r = i * 8 + kr, key = kt * kFK + r;
+      float4v lo = klo[i], hi = khi[i];
+      if (tabk != nullptr) {
+        const float4v* tp = (const float4v*)(tabk + (int64_t)(key < Lk ? key : Lk - 1) * 32 + 4 * c8);
+        const float4v t0 = tp[0], t1 = tp[1];
+        const float cc[4] = {t0[0], t0[2], t1[0], t1[2]}, ss[4] = {t0[1], t0[3], t1[1], t1[3]};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float x0 = lo[e], x1 = hi[e];
+          lo[e] = fmaf(-x1, ss[e], x0 * cc[e]);
+          hi[e] = fmaf(x0, ss[e], x1 * cc[e]);
+        }
+      }
+      *(float4v*)(kb + kslot(r, c8)) = lo;
+      *(float4v*)(kb + kslot(r, c8 + 8)) = hi;
+    }
+  };
+
+  float16v o[2];
+#pragma unroll
+  for (int d = 0; d < 2; d++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) o[d][r] = 0.f;
+  float m = -INFINITY, l = 0.f;
+
+  int i0 = wave;
+  if (i0 < nt) load_k(todo[i0] >> 1);
+  for (; i0 < nt; i0 += kFW) {
+    const int ent = __builtin_amdgcn_readfirstlane((int)todo[i0]), kt = ent >> 1, k0 = kt * kFK;
+    store_k(kt);
+    // the tile is this wave's own: its LDS stores and loads only need to stay
+    // in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // V of the tile, the next tile's K
+    float v[2][16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int key = k0 + 8 * (r >> 2) + 4 * lg + (r & 3);
+      const float* p = Vb + (int64_t)(key < Lk ? key : Lk - 1) * vs.s[2] + l32;
+      v[0][r] = p[0];
+      v[1][r] = p[32];
+    }
+    if (i0 + kFW < nt) load_k(todo[i0 + kFW] >> 1);
+
+    float16v s;
+#pragma unroll
+    for (int r = 0; r < 16; r++) s[r] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float4v kf = *(const float4v*)(kb + kslot(l32, 2 * i + lg));
+#pragma unroll
+      for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qf[i][e], s, 0, 0, 0);
+    }
+    // (the next store_k must not overtake these reads)
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+
+    const bool mixed = ent & 1;
+    const uint8_t* mrow = mask == nullptr ? nullptr
+                                          : mask + b * ms.s[0] + h * ms.s[1] + (int64_t)(q < Lq ? q : Lq - 1) * ms.s[2];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      s[r] *= scale;
+      if (mixed) {
+        const int key = k0 + 8 * (r >> 2) + 4 * lg + (r & 3);
+        const bool vis = key < Lk && (mrow == nullptr || mrow[(int64_t)key * ms.s[3]] != 0);
+        s[r] = vis ? s[r] : -INFINITY;
+      }
+      mx = fmaxf(mx, s[r]);
+    }
+    mx = max_xor32(mx);
+    const float mnew = fmaxf(m, mx);
+    const float mc = mnew == -INFINITY ? 0.f : mnew;  // no visible key yet: every weight is exp(-inf) = 0
+    const float alpha = expf(m - mc);
+    m = mnew;
+    float sum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      s[r] = expf(s[r] - mc);
+      sum += s[r];
+    }
+    l = l * alpha + sum;
+    if (!__all(alpha == 1.0f)) {
+#pragma unroll
+      for (int d = 0; d < 2; d++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[d][r] *= alpha;
+    }
+    // A non-finite V must not reach a query whose weight for that key is 0
+    // (hidden, or exp underflowed), as 0 * inf in the product would: such a
+    // tile is added key by key, zero weights skipped.
+    float fin = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; r++) fin += v[0][r] * 0.f + v[1][r] * 0.f;
+    if (__any(fin != 0.f)) {  // 0 * finite = 0, 0 * (inf or NaN) = NaN
+#pragma unroll
+      for (int r = 0; r < 16; r++) kb[(8 * (r >> 2) + 4 * lg + (r & 3)) * 32 + l32] = s[r];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+      for (int j = 0; j < kFK; j++) {
+        const float p = kb[j * 32 + l32];
+        if (p == 0.f) continue;  // keys past Lk among them
+        const float* vp = Vb + (int64_t)(k0 + j) * vs.s[2] + 4 * lg;
+#pragma unroll
+        for (int d = 0; d < 2; d++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) o[d][r] = fmaf(p, vp[32 * d + 8 * (r >> 2) + (r & 3)], o[d][r]);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+#pragma unroll
+      for (int d = 0; d < 2; d++) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[d][r], s[r], o[d], 0, 0, 0);
+  }
+
+  // merge the waves' outputs: weights exp(m_w - max); wave w finishes
+  // registers [8 w, 8 w + 8) of the 32
+  l = sum_xor32(l);
+  if (lg == 0) {
+    part_m[wave][l32] = m;
+    part_l[wave][l32] = l;
+  }
+  __syncthreads();  // every wave is done with its K tile
+#pragma unroll
+  for (int d = 0; d < 2; d++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) buf[wave][(d * 16 + r) * 64 + lane] = o[d][r];
+  __syncthreads();
+  float mt = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < kFW; w++) mt = fmaxf(mt, part_m[w][l32]);
+  const float mc = mt == -INFINITY ? 0.f : mt;
+  float wt[kFW], lt = 0.f;
+#pragma unroll
+  for (int w = 0; w < kFW; w++) {
+    wt[w] = expf(part_m[w][l32] - mc);
+    lt += part_l[w][l32] * wt[w];
+  }
+  const float inv = 1.0f / lt;
+  if (q >= Lq) return;
+  float* op = O + b * os.s[0] + h * os.s[1] + (int64_t)q * os.s[2];
+#pragma unroll
+  for (int r4 = 0; r4 < 2; r4++) {
+    const int x = wave * 8 + r4 * 4;  // register x: column 32 * (x / 16) + 8 * (x % 16 / 4) + 4 * lg
+    float4v ov;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      float a = 0.f;
+#pragma unroll
+      for (int w = 0; w < kFW; w++) a += buf[w][(x + e) * 64 + lane] * wt[w];
+      ov[e] = a * inv;
+    }
+    *(float4v*)(op + 32 * (x >> 4) + 8 * ((x & 15) >> 2) + 4 * lg) = ov;
+  }
+}
+
 // ------------------------------------------------------------------ SIMT kernel (any dtype / D)
 
 // One wave per query row: scores for every key into LDS, softmax in f32,
@@ -691,6 +967,18 @@ static bool sdpa_takes_mfma(int dt, uintptr_t q, const int64_t* qs, uintptr_t k,
          ks[2] < (1 << 24) && vs[2] >= 0 && vs[2] < (1 << 24);
 }
 
+// The f32 MFMA kernel's conditions: D = 64, unit inner strides, 16-byte
+// aligned rows, and no more keys than sdpa_simt takes.  Any mask goes: one
+// without a summary (it varies over heads) is read for every tile.
+static bool sdpa_takes_f32(int dt, uintptr_t q, const int64_t* qs, uintptr_t k, const int64_t* ks, uintptr_t v,
+                           const int64_t* vs, uintptr_t o, const int64_t* os, int64_t Lk, int64_t D) {
+  auto rows16 = [](uintptr_t p, const int64_t* s) {
+    return p % 16 == 0 && s[3] == 1 && s[0] % 4 == 0 && s[1] % 4 == 0 && s[2] % 4 == 0;
+  };
+  return dt == HB_F32 && D == 64 && Lk > 0 && rows16(q, qs) && rows16(k, ks) && v % 4 == 0 && vs[3] == 1 &&
+         rows16(o, os) && (Lk + D) * 4 <= 160 * 1024;
+}
+
 // The argument checks every sdpa entry point makes before it launches
 // anything.
 static void sdpa_check(int dt, const int64_t* qs, const int64_t* ks, const int64_t* vs, uintptr_t mask,
@@ -752,6 +1040,16 @@ static void sdpa_impl(uintptr_t ctx, int dt, uintptr_t q, const int64_t* qs, uin
                                             (int)Lk, sl2, tq, tk, pK, nqt, (int)H);
     check_launch("hb_sdpa");
     if (tmp) pool_free(ctx, tmp);
+  } else if (sdpa_takes_f32(dt, q, qs, k, ks, v, vs, o, os, Lk, D)) {
+    const int nqt = (int)((Lq + kFQ - 1) / kFQ);
+    const int64_t nblk = (int64_t)nqt * H * B;
+    HB_REQUIRE(nblk < ((int64_t)1 << 31), "hb_sdpa: too many (batch, head, query tile) blocks");
+    // (a caller's summary only describes a mask that does not vary over heads)
+    const uint8_t* info = mask && ms[1] == 0 ? (const uint8_t*)mask_info : nullptr;
+    sdpa_f32_mfma<<<(unsigned)nblk, kFW * 64, 0, st>>>((const float*)q, Qs, (const float*)k, Ks, (const float*)v, Vs,
+                                                       (const uint8_t*)mask, Ms, info, (float*)o, Os, (int)Lq, (int)Lk,
+                                                       scale, tq, tk, nqt, (int)H);
+    check_launch("hb_sdpa(f32)");
   } else {
     size_t lds = sizeof(float) * (size_t)(Lk + D);
     HB_REQUIRE(lds <= 160 * 1024, "hb_sdpa: sequence too long for the generic kernel");
