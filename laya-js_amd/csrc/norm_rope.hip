@@ -158,6 +158,57 @@ __global__ __launch_bounds__(kLnNT) void layernorm_panel_kernel(const uint16_t* 
   }
 }
 
+// f32 rows of 256 * G values: one row per wave, held in registers (16-byte
+// loads), so it is read once.  Memory-bound; the generic kernel below reads
+// the row three times, 4 bytes a lane, and each pass waits for the last.
+template <int G, int PK>
+__global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restrict__ x, int64_t ldx,
+                                                            const void* __restrict__ w, const void* __restrict__ b,
+                                                            float* __restrict__ y, int64_t rows, float eps) {
+  constexpr int D = 256 * G;
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const float* xr = x + row * ldx;
+  float4v v[G];
+  float s = 0.0f;
+#pragma unroll
+  for (int g = 0; g < G; g++) v[g] = *(const float4v*)(xr + (g * 64 + lane) * 4);
+#pragma unroll
+  for (int g = 0; g < G; g++) s += (v[g][0] + v[g][1]) + (v[g][2] + v[g][3]);
+  const float mean = wave_sum(s) / (float)D;
+  float q = 0.0f;
+#pragma unroll
+  for (int g = 0; g < G; g++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const float d = v[g][e] - mean;
+      q += d * d;
+    }
+  const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)D + eps);
+  float* yr = y + row * D;
+#pragma unroll
+  for (int g = 0; g < G; g++) {
+    const int c = (g * 64 + lane) * 4;
+    float wv[4] = {1.f, 1.f, 1.f, 1.f}, bv[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (PK != 0) {
+      if (w) load4_param<PK>(w, c, wv);
+      if (b) load4_param<PK>(b, c, bv);
+    }
+    float4v o;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      float t = (v[g][e] - mean) * rstd;
+      if constexpr (PK != 0) {
+        if (w) t *= wv[e];
+        if (b) t += bv[e];
+      }
+      o[e] = t;
+    }
+    *(float4v*)(yr + c) = o;
+  }
+}
+
 // Generic: any dtype and width; the row is re-read for each pass.
 __global__ __launch_bounds__(256) void layernorm_kernel(int dt_x, const void* __restrict__ x, int64_t ldx, int dt_w,
                                                         const void* __restrict__ w, const void* __restrict__ b,
@@ -212,10 +263,35 @@ static int ln_param_kind(int dt_w, uintptr_t w, uintptr_t b) {
 }
 
 // The 16-bit kernels' conditions (besides the output's).
-static bool ln_vec_ok(int dt_x, uintptr_t x, int64_t ldx, int pk, uintptr_t w, uintptr_t b, int64_t D) {
+static bool ln_rows_ok(uintptr_t x, int64_t ldx, int pk, uintptr_t w, uintptr_t b, int64_t D, int es) {
   const int64_t pal = pk == 3 ? 16 : 8;  // parameter alignment the 4-wide loads need
-  return (dt_x == HB_F16 || dt_x == HB_BF16) && D % 256 == 0 && D <= 2048 && ldx % 8 == 0 && x % 16 == 0 &&
-         pk >= 0 && w % pal == 0 && b % pal == 0;
+  return D % 256 == 0 && D <= 2048 && ldx * es % 16 == 0 && x % 16 == 0 && pk >= 0 && w % pal == 0 && b % pal == 0;
+}
+static bool ln_vec_ok(int dt_x, uintptr_t x, int64_t ldx, int pk, uintptr_t w, uintptr_t b, int64_t D) {
+  return (dt_x == HB_F16 || dt_x == HB_BF16) && ln_rows_ok(x, ldx, pk, w, b, D, 2);
+}
+
+// launch(G, PK) with both as compile-time constants (G = 1..8, PK = 0..3)
+template <class Launch>
+static void ln_dispatch(int G, int pk, Launch&& launch) {
+  auto by_g = [&](auto pc) {
+    switch (G) {
+      case 1: launch(std::integral_constant<int, 1>{}, pc); break;
+      case 2: launch(std::integral_constant<int, 2>{}, pc); break;
+      case 3: launch(std::integral_constant<int, 3>{}, pc); break;
+      case 4: launch(std::integral_constant<int, 4>{}, pc); break;
+      case 5: launch(std::integral_constant<int, 5>{}, pc); break;
+      case 6: launch(std::integral_constant<int, 6>{}, pc); break;
+      case 7: launch(std::integral_constant<int, 7>{}, pc); break;
+      default: launch(std::integral_constant<int, 8>{}, pc); break;
+    }
+  };
+  switch (pk) {
+    case 0: by_g(std::integral_constant<int, 0>{}); break;
+    case 1: by_g(std::integral_constant<int, 1>{}); break;
+    case 2: by_g(std::integral_constant<int, 2>{}); break;
+    default: by_g(std::integral_constant<int, 3>{}); break;
+  }
 }
 
 static void launch_ln16(bool panel, hipStream_t st, bool bf, int pk, const uint16_t* x, int64_t ldx, uintptr_t w,
@@ -240,24 +316,16 @@ static void launch_ln16(bool panel, hipStream_t st, bool bf, int pk, const uint1
       kern<<<(unsigned)((rows + 7) / 8), 256, 0, st>>>(x, ldx, (const void*)w, (const void*)b, y, rows, D, eps);
     }
   };
-  auto by_g = [&](auto pc) {
-    switch (G) {
-      case 1: launch(std::integral_constant<int, 1>{}, pc); break;
-      case 2: launch(std::integral_constant<int, 2>{}, pc); break;
-      case 3: launch(std::integral_constant<int, 3>{}, pc); break;
-      case 4: launch(std::integral_constant<int, 4>{}, pc); break;
-      case 5: launch(std::integral_constant<int, 5>{}, pc); break;
-      case 6: launch(std::integral_constant<int, 6>{}, pc); break;
-      case 7: launch(std::integral_constant<int, 7>{}, pc); break;
-      default: launch(std::integral_constant<int, 8>{}, pc); break;
-    }
-  };
-  switch (pk) {
-    case 0: by_g(std::integral_constant<int, 0>{}); break;
-    case 1: by_g(std::integral_constant<int, 1>{}); break;
-    case 2: by_g(std::integral_constant<int, 2>{}); break;
-    default: by_g(std::integral_constant<int, 3>{}); break;
-  }
+  ln_dispatch(G, pk, launch);
+}
+
+// f32 in and out (the conditions of ln_vec_ok with 16-byte f32 rows)
+static void launch_ln32(hipStream_t st, int pk, const float* x, int64_t ldx, uintptr_t w, uintptr_t b, float* y,
+                        int64_t rows, int D, float eps) {
+  ln_dispatch(D / 256, pk, [&](auto gc, auto pc) {
+    layernorm_f32_kernel<decltype(gc)::value, decltype(pc)::value><<<(unsigned)((rows + 3) / 4), 256, 0, st>>>(
+        x, ldx, (const void*)w, (const void*)b, y, rows, eps);
+  });
 }
 
 }  // namespace hb
@@ -275,6 +343,8 @@ int hb_layernorm(uintptr_t ctx, int dt_x, uintptr_t x, int64_t ldx, int dt_w, ui
   const int pk = ln_param_kind(dt_w, w, b);
   if (dt_y == dt_x && ln_vec_ok(dt_x, x, ldx, pk, w, b, D) && y % 16 == 0) {
     launch_ln16(false, st, dt_x == HB_BF16, pk, (const uint16_t*)x, ldx, w, b, (uint16_t*)y, rows, (int)D, eps);
+  } else if (dt_x == HB_F32 && dt_y == HB_F32 && ln_rows_ok(x, ldx, pk, w, b, D, 4) && y % 16 == 0) {
+    launch_ln32(st, pk, (const float*)x, ldx, w, b, (float*)y, rows, (int)D, eps);
   } else {
     layernorm_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, st>>>(dt_x, (const void*)x, ldx, dt_w, (const void*)w,
                                                                  (const void*)b, dt_y, (void*)y, rows, D, eps);
