@@ -20,6 +20,11 @@
 // Backend.rope.  The output is written row-major or, for the attention output
 // projection, in the panel order of the GEMM's X operand.
 //
+// sdpa32_ring: the same for longer sequences and masks that every query
+// shares, 32 queries per wave on v_mfma_f32_32x32x16 (sdpa_impl says where the
+// line lies).  V goes to LDS by direct loads and is transposed by the LDS read;
+// K likewise, or through registers where RoPE rotates it on the way.
+//
 // sdpa_f32_mfma: the f32 path for head dim 64, on v_mfma_f32_32x32x2_f32.
 //
 // sdpa_simt: the fallback for other head dims / layouts.
@@ -61,6 +66,12 @@ constexpr int kMaxKeyTiles = 1024;  // Lk <= 65536 on the MFMA path
 
 // ------------------------------------------------------------------ mask summary
 
+// 4 mask bytes (any nonzero byte is true): bit 7 of each byte set iff the
+// byte is nonzero (no carries between bytes)
+__device__ __forceinline__ uint32_t mask_nz(uint32_t w) {
+  return (((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u;
+}
+
 // Class of every (batch, 16-query group, 64-key tile) block of a bool mask:
 // 0 = no visible key (skipped), 1 = every key visible (no mask reads),
 // 2 = mixed or running past Lk (per-element mask).  One byte per group, the
@@ -68,41 +79,35 @@ constexpr int kMaxKeyTiles = 1024;  // Lk <= 65536 on the MFMA path
 // + group].  Computed once per mask tensor and reused by every layer that
 // attends with it; the attention kernel skips a key tile for a wave whose
 // group has class 0 and stages it only if some group needs it.
-__global__ __launch_bounds__(256) void mask_class_kernel(const uint8_t* __restrict__ mask, S4 ms, int Lq, int Lk,
-                                                         int nqt, int nkt, uint8_t* __restrict__ cls, int vec) {
-  __shared__ int anyg[kNW], allg[kNW];
+// One wave per 16-query group: a lane takes 16 bytes of one of the group's rows
+// (unaligned loads, so any row length does), and two ballots give the class.
+// Bound by reading the mask once; measured on B = 3, T = 333, where the rows
+// are not 16-byte aligned: 11.2 -> 5.2 us against a byte per thread and LDS
+// atomics.
+__global__ __launch_bounds__(kNW * 64) void mask_class_kernel(const uint8_t* __restrict__ mask, S4 ms, int Lq, int Lk,
+                                                         int nqt, int nkt, uint8_t* __restrict__ cls) {
   const int kt = blockIdx.x, qt = blockIdx.y, b = blockIdx.z;
-  const int q0 = qt * kBQ, k0 = kt * kBK;
-  const int nq = min(kBQ, Lq - q0), nk = min(kBK, Lk - k0);
-  const bool bcast = ms.s[2] == 0;  // a [B,1,1,L] mask has one row for every query
-  if (threadIdx.x < kNW) {
-    anyg[threadIdx.x] = 0;
-    allg[threadIdx.x] = 1;
-  }
-  __syncthreads();
-  if (vec && nk == kBK) {
-    // 16-byte row chunks: rows x 4 chunks
-    for (int i = threadIdx.x; i < nq * 4; i += blockDim.x) {
-      const int q = i >> 2, c = i & 3;
-      const uint4v w = *(const uint4v*)(mask + b * ms.s[0] + (int64_t)(bcast ? 0 : q0 + q) * ms.s[2] + k0 + c * 16);
-      // any byte nonzero <=> word != 0; all visible when every byte == 1
-      const uint32_t o = w.x | w.y | w.z | w.w, a = w.x & w.y & w.z & w.w;
-      if (o != 0) atomicOr(&anyg[q >> 4], 1);
-      if (a != 0x01010101u) atomicAnd(&allg[q >> 4], 0);
-    }
-  } else {
-    for (int i = threadIdx.x; i < nq * nk; i += blockDim.x) {
-      const int q = i / nk, k = i - q * nk;
-      const uint8_t m = mask[b * ms.s[0] + (int64_t)(bcast ? 0 : q0 + q) * ms.s[2] + (int64_t)(k0 + k) * ms.s[3]];
-      if (m != 0) atomicOr(&anyg[q >> 4], 1);
-      else atomicAnd(&allg[q >> 4], 0);
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int k0 = kt * kBK, nk = min(kBK, Lk - k0), c = (lane & 3) * 16;
+  const int q = qt * kBQ + g * 16 + (lane >> 2);
+  bool any = false, all = true;
+  if (q < Lq && c < nk) {
+    const uint8_t* p = mask + b * ms.s[0] + (int64_t)q * ms.s[2] + (int64_t)(k0 + c) * ms.s[3];
+    if (ms.s[3] == 1 && c + 16 <= nk) {
+      uint32_t w[4];
+      __builtin_memcpy(w, p, 16);
+      any = (w[0] | w[1] | w[2] | w[3]) != 0;
+      all = (mask_nz(w[0]) & mask_nz(w[1]) & mask_nz(w[2]) & mask_nz(w[3])) == 0x80808080u;
+    } else {
+      for (int e = 0; e < 16 && c + e < nk; e++) {
+        const bool v = p[(int64_t)e * ms.s[3]] != 0;
+        any |= v;
+        all &= v;
+      }
     }
   }
-  __syncthreads();
-  if (threadIdx.x < kNW) {
-    const int g = threadIdx.x;
-    cls[(((int64_t)b * nqt + qt) * nkt + kt) * kNW + g] = !anyg[g] ? 0 : (allg[g] && nk == kBK ? 1 : 2);
-  }
+  const bool gany = __ballot(any) != 0, gall = __ballot(!all) == 0;
+  if (lane == 0) cls[(((int64_t)b * nqt + qt) * nkt + kt) * kNW + g] = !gany ? 0 : (gall && nk == kBK ? 1 : 2);
 }
 
 static size_t mask_info_bytes(int64_t B, int64_t Lq, int64_t Lk) {
@@ -113,8 +118,7 @@ static size_t mask_info_bytes(int64_t B, int64_t Lq, int64_t Lk) {
 static void launch_mask_info(hipStream_t st, const uint8_t* mask, const S4& ms, int64_t B, int64_t Lq, int64_t Lk,
                              uint8_t* info) {
   int nqt = (int)((Lq + kBQ - 1) / kBQ), nkt = (int)((Lk + kBK - 1) / kBK);
-  int vec = ms.s[3] == 1 && ((uintptr_t)mask % 16 == 0) && ms.s[0] % 16 == 0 && ms.s[2] % 16 == 0;
-  mask_class_kernel<<<dim3(nkt, nqt, (unsigned)B), 256, 0, st>>>(mask, ms, (int)Lq, (int)Lk, nqt, nkt, info, vec);
+  mask_class_kernel<<<dim3(nkt, nqt, (unsigned)B), kNW * 64, 0, st>>>(mask, ms, (int)Lq, (int)Lk, nqt, nkt, info);
 }
 
 // ------------------------------------------------------------------ MFMA kernel (D = 64)
@@ -137,22 +141,16 @@ __device__ __forceinline__ uint32_t fromf(float v) {
   return BF16 ? f32_to_bf16(v) : f32_to_f16_bits(v);
 }
 
-// Two f32 values packed as 16-bit (f16: v_cvt_pk_f16_f32; bf16: RNE).
+// Two f32 values packed as 16-bit (v_cvt_pk_f16_f32 / v_cvt_pk_bf16_f32: RNE).
 template <bool BF16>
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
+  typedef float float2v __attribute__((ext_vector_type(2)));
   if constexpr (BF16) {
-    return (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2v){a, b}, bf16x2));
   } else {
-    typedef float float2v __attribute__((ext_vector_type(2)));
-    half2v h = __builtin_convertvector((float2v){a, b}, half2v);
-    return __builtin_bit_cast(uint32_t, h);
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2v){a, b}, half2v));
   }
-}
-
-// 4 mask bytes (any nonzero byte is true): bit 7 of each byte set iff the
-// byte is nonzero (no carries between bytes)
-__device__ __forceinline__ uint32_t mask_nz(uint32_t w) {
-  return (((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u;
 }
 
 // Cross-lane exchanges for the 4 lanes that hold one query (lane, lane ^ 16,
@@ -212,24 +210,29 @@ __device__ __forceinline__ void load_cs(const float2* __restrict__ tab, int pos,
   }
 }
 
+// Rotates a loaded chunk pair by RoPE, rounding to the storage type like a
+// separate Backend.rope.
+template <bool BF16>
+__device__ __forceinline__ void rot_pair(uint4v& lo, uint4v& hi, const float2 (&cs)[8]) {
+  uint32_t* l = (uint32_t*)&lo;
+  uint32_t* h = (uint32_t*)&hi;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const float2 c0 = cs[2 * e], c1 = cs[2 * e + 1];
+    float x0a = tof<BF16>(l[e] & 0xffff), x0b = tof<BF16>(l[e] >> 16);
+    float x1a = tof<BF16>(h[e] & 0xffff), x1b = tof<BF16>(h[e] >> 16);
+    l[e] = pack2<BF16>(pin_f32(fmaf(-x1a, c0.y, x0a * c0.x)), pin_f32(fmaf(-x1b, c1.y, x0b * c1.x)));
+    h[e] = pack2<BF16>(pin_f32(fmaf(x0a, c0.y, x1a * c0.x)), pin_f32(fmaf(x0b, c1.y, x1b * c1.x)));
+  }
+}
+
 // Rotates a loaded chunk pair by RoPE (when `rot`) with the pairs' cos / sin,
 // rounding to the storage type like a separate Backend.rope, and writes it
 // to the swizzled [rows][64] LDS tile.
 template <bool BF16, bool KSWZ = false>
 __device__ __forceinline__ void store_pair(uint4v lo, uint4v hi, bool rot, int c, const float2 (&cs)[8],
                                            uint16_t* lds, int row) {
-  if (rot) {
-    uint32_t* l = (uint32_t*)&lo;
-    uint32_t* h = (uint32_t*)&hi;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const float2 c0 = cs[2 * e], c1 = cs[2 * e + 1];
-      float x0a = tof<BF16>(l[e] & 0xffff), x0b = tof<BF16>(l[e] >> 16);
-      float x1a = tof<BF16>(h[e] & 0xffff), x1b = tof<BF16>(h[e] >> 16);
-      l[e] = pack2<BF16>(pin_f32(fmaf(-x1a, c0.y, x0a * c0.x)), pin_f32(fmaf(-x1b, c1.y, x0b * c1.x)));
-      h[e] = pack2<BF16>(pin_f32(fmaf(x0a, c0.y, x1a * c0.x)), pin_f32(fmaf(x0b, c1.y, x1b * c1.x)));
-    }
-  }
+  if (rot) rot_pair<BF16>(lo, hi, cs);
   *(uint4v*)(lds + (KSWZ ? k_swz(row, c) : qk_swz(row, c))) = lo;
   *(uint4v*)(lds + (KSWZ ? k_swz(row, c + 4) : qk_swz(row, c + 4))) = hi;
 }
@@ -355,8 +358,8 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void s
 #pragma unroll
       for (int t = 0; t < 2; t++) {
         const int kbase = k0 + 32 * t + 8 * g;
-        if (mask_vec && kbase + 8 <= Lk) {
-          mw[qb][t] = *(const uint2v*)(mrow + kbase);
+        if (mask_vec && kbase + 8 <= Lk) {  // (rows of any alignment)
+          __builtin_memcpy(&mw[qb][t], mrow + kbase, 8);
         } else {
           uint32_t w0 = 0, w1 = 0;
 #pragma unroll
@@ -588,6 +591,424 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void s
       *(uint2v*)(op + d * dstep) = w;
     }
   }
+}
+
+// ------------------------------------------------------------------ 32-query MFMA kernel
+
+// 16 bytes per lane from buffer `rs` at byte offset `voff` straight into LDS:
+// lane l fills [lds + 16 l, + 16); an offset past the buffer's records writes
+// zeros.  Inline asm, so that the compiler neither holds later LDS reads of the
+// other buffer behind it nor counts it in its own waits (an extra load in
+// flight only makes those stronger); the caller waits for it (vmcnt(0)).
+__device__ __forceinline__ void buffer_to_lds16(const uint4v& rs, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
+               : "memory");
+}
+typedef short short4t __attribute__((ext_vector_type(4)));
+// Transposing LDS read: within 16 lanes, lanes 4r .. 4r + 3 point at 4 x 4
+// consecutive values of row r; lane c gets column c's 4 rows.
+__device__ __forceinline__ uint2v lds_tr16(const uint16_t* p) {
+  const short4t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4t*)p);
+  return __builtin_bit_cast(uint2v, v);
+}
+template <bool BF16>
+__device__ __forceinline__ float16v mfma32x16(const uint4v& a, const uint4v& b, float16v c) {
+  if constexpr (BF16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                   0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0,
+                                                  0);
+}
+
+// chunk c (8 values) of row r of a [64][64] K or V tile sits at c ^ kv_f(r): a
+// 16-lane pass of the K fragment reads (16 rows, one chunk) and of the V
+// transpose reads (4 rows, 4 chunks) covers all 64 banks
+__device__ __forceinline__ int kv_f(int r) { return (((r >> 1) & 1) << 2) | ((r >> 2) & 3); }
+
+// K [B, H, Lk, 64] rotated by RoPE into contiguous [B, H, Lk, 64]: one thread
+// per chunk pair (c, c + 4) of a row.  Bandwidth-bound; blocks take 64 rows of
+// every (b, h) in turn, so the RoPE table's rows stay in L2.
+template <bool BF16>
+__global__ __launch_bounds__(256) void rope_k_kernel(const uint16_t* __restrict__ K, S4 ks, uint16_t* __restrict__ Y,
+                                                     int Lk, int nh, int nbh, const float2* __restrict__ tab) {
+  const int bh = blockIdx.x % nbh, r = (blockIdx.x / nbh) * 64 + (threadIdx.x >> 2), c = threadIdx.x & 3;
+  if (r >= Lk) return;
+  const uint16_t* kp = K + (bh / nh) * ks.s[0] + (bh % nh) * ks.s[1] + (int64_t)r * ks.s[2];
+  uint4v lo, hi;
+  float2 cs[8];
+  load_pair(kp, true, c, lo, hi);
+  load_cs(tab + (int64_t)r * 32, 0, c, cs);
+  rot_pair<BF16>(lo, hi, cs);
+  uint16_t* yp = Y + ((int64_t)bh * Lk + r) * 64;
+  *(uint4v*)(yp + 8 * c) = lo;
+  *(uint4v*)(yp + 8 * (c + 4)) = hi;
+}
+
+// One wave's state: 32 queries (lane l holds query l % 32; the lane halves
+// split its columns of Q and O and its keys).
+struct Wave32 {
+  uint4v qf[4];   // chunk 2 s + lg of the query (columns 16 s + 8 lg ..) per MFMA step s
+  float16v o[2];  // O^T: columns 32 d + 8 (r / 4) + 4 lg + r % 4
+  float m, l;     // raw (unscaled) row max, sum of the lane's weights
+};
+
+// Loads the wave's queries and, with a table, rotates them, rounded as a
+// separate Backend.rope stores them.
+template <bool BF16>
+__device__ __forceinline__ void wave32_init(Wave32& w, const uint16_t* qrow, const float2* tab, int pos, int lg) {
+#pragma unroll
+  for (int s = 0; s < 4; s++) w.qf[s] = *(const uint4v*)(qrow + 8 * lg + 16 * s);
+  if (tab != nullptr) {
+    const float4v* tp = (const float4v*)(tab + (int64_t)pos * 32 + 8 * lg);
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      float2 cs[8];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float4v v = tp[8 * s + e];
+        cs[2 * e] = float2{v[0], v[1]};
+        cs[2 * e + 1] = float2{v[2], v[3]};
+      }
+      rot_pair<BF16>(w.qf[s], w.qf[s + 2], cs);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < 2; d++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) w.o[d][r] = 0.f;
+  w.m = -INFINITY;
+  w.l = 0.f;
+}
+
+// LDS element offsets of a lane's fragment reads within a [64][64] tile: K
+// chunk 2 s + lg of row l32 (+ 2048 for the second 32 keys); V transpose
+// read of keys 16 t + 8 u + 4 lg .., columns 32 d .. (+ 1024 t).
+struct Frag32 {
+  int ka[4], va[2][2];
+};
+__device__ __forceinline__ Frag32 frag32(int lane) {
+  Frag32 f;
+  const int l32 = lane & 31, lg = lane >> 5, j16 = lane & 15, vrow = 4 * lg + (j16 >> 2);
+#pragma unroll
+  for (int s = 0; s < 4; s++) f.ka[s] = l32 * 64 + (((2 * s + lg) ^ kv_f(l32)) << 3);
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int d = 0; d < 2; d++) {
+      const int r = 8 * u + vrow, c = 4 * d + 2 * ((lane >> 4) & 1) + ((j16 & 3) >> 1);
+      f.va[u][d] = r * 64 + ((c ^ kv_f(r)) << 3) + 4 * (j16 & 1);
+    }
+  return f;
+}
+
+// One 64-key tile (keys k0 ..) for the wave's queries: scores, mask (`mixed`),
+// online softmax, O += P . V.  mrow: the lane's mask row, or null (only the
+// bound Lk hides keys); mask_vec: its rows are contiguous and 16-byte aligned,
+// and lane half lg fetches the 32 bytes of key block lg, the halves swapping
+// words afterwards; otherwise a lane's own words (keys 32 kb + 8 j + 4 lg ..).
+template <bool BF16>
+__device__ __forceinline__ void wave32_tile(Wave32& w, const Frag32& f, const uint16_t* Kc, const uint16_t* Vc, int k0,
+                                            int Lk, bool mixed, const uint8_t* mrow, int64_t ms3, int mask_vec,
+                                            float scale_log2, int lg) {
+  const bool vec = mask_vec && k0 + kBK <= Lk;
+  uint32_t mw[8];
+  if (mixed && mrow != nullptr) {
+    if (vec) {
+      const uint4v a = *(const uint4v*)(mrow + k0 + 32 * lg), c = *(const uint4v*)(mrow + k0 + 32 * lg + 16);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        mw[e] = a[e];
+        mw[4 + e] = c[e];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const int key = k0 + 32 * (i >> 2) + 8 * (i & 3) + 4 * lg;
+        uint32_t v = 0;
+        if (ms3 == 1 && key + 4 <= Lk) {
+          __builtin_memcpy(&v, mrow + key, 4);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            if (key + e < Lk && mrow[(int64_t)(key + e) * ms3] != 0) v |= 1u << (8 * e);
+        }
+        mw[i] = v;
+      }
+    }
+  }
+  float16v st[2];
+#pragma unroll
+  for (int kb = 0; kb < 2; kb++) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) st[kb][r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; s++) st[kb] = mfma32x16<BF16>(*(const uint4v*)(Kc + f.ka[s] + kb * 2048), w.qf[s], st[kb]);
+  }
+  if (mixed) {
+    uint32_t x[8];
+    if (mrow == nullptr) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) x[i] = 0x01010101u;
+    } else if (vec) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const auto y = __builtin_amdgcn_permlane32_swap(mw[2 * j], mw[2 * j + 1], false, false);
+        x[j] = (uint32_t)y[0];
+        x[4 + j] = (uint32_t)y[1];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; i++) x[i] = mw[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      // bit 7 of byte e: key visible; a hidden score becomes -inf
+      uint32_t vis = mask_nz(x[i]);
+      const int left = Lk - (k0 + 32 * (i >> 2) + 8 * (i & 3) + 4 * lg);
+      vis &= left >= 4 ? ~0u : (left <= 0 ? 0u : 0xffffffffu >> (8 * (4 - left)));
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const uint32_t mk = (uint32_t)__builtin_amdgcn_sbfe((int)vis, 8 * e + 7, 1);
+        const float sv = st[i >> 2][4 * (i & 3) + e];
+        st[i >> 2][4 * (i & 3) + e] = __uint_as_float((__float_as_uint(sv) & mk) | (~mk & 0xff800000u));
+      }
+    }
+  }
+  float mx = -INFINITY;
+#pragma unroll
+  for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) mx = fmaxf(mx, st[kb][r]);
+  mx = max_xor32(mx);
+  const float mnew = fmaxf(w.m, mx);
+  const float mc = mnew == -INFINITY ? 0.f : mnew * scale_log2;
+  const float alpha = __builtin_amdgcn_exp2f(w.m * scale_log2 - mc);
+  w.m = mnew;
+  float psum = 0.f;
+  uint4v pf[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    uint32_t pk[4];
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const float p0 = __builtin_amdgcn_exp2f(fmaf(st[t >> 1][8 * (t & 1) + e], scale_log2, -mc));
+      const float p1 = __builtin_amdgcn_exp2f(fmaf(st[t >> 1][8 * (t & 1) + e + 1], scale_log2, -mc));
+      psum += p0 + p1;
+      pk[e >> 1] = pack2<BF16>(p0, p1);
+    }
+    pf[t] = uint4v{pk[0], pk[1], pk[2], pk[3]};
+  }
+  w.l = w.l * alpha + psum;
+  if (!__all(alpha == 1.0f)) {  // rescale O only when some row max of this wave moved
+#pragma unroll
+    for (int d = 0; d < 2; d++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) w.o[d][r] *= alpha;
+  }
+#pragma unroll
+  for (int t = 0; t < 4; t++)
+#pragma unroll
+    for (int d = 0; d < 2; d++) {
+      const uint2v v0 = lds_tr16(Vc + f.va[0][d] + t * 1024), v1 = lds_tr16(Vc + f.va[1][d] + t * 1024);
+      w.o[d] = mfma32x16<BF16>(uint4v{v0.x, v0.y, v1.x, v1.y}, pf[t], w.o[d]);
+    }
+}
+
+// Normalises and stores query q: 4 consecutive columns 32 d + 8 j + 4 lg per 8
+// bytes, strided [B, H, Lq, D], or (pK > 0) in panel order of the [B*Lq, pK]
+// matrix whose rows hold the heads side by side: 16-column block 4 h + 2 d +
+// j / 2, half j % 2.
+template <bool BF16>
+__device__ __forceinline__ void wave32_store(const Wave32& w, uint16_t* O, const S4& os, int pK, int b, int h, int q,
+                                             int Lq, int lg) {
+  const float inv = 1.0f / sum_xor32(w.l);
+  if (q >= Lq) return;
+  const int64_t mrw = (int64_t)b * Lq + q;
+  uint16_t* op = pK > 0 ? O + ((mrw >> 5) * (pK >> 4) + 4 * h) * 512 + (mrw & 31) * 8 + 4 * lg
+                        : O + b * os.s[0] + h * os.s[1] + (int64_t)q * os.s[2] + 4 * lg;
+#pragma unroll
+  for (int d = 0; d < 2; d++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      uint2v x;
+      x.x = pack2<BF16>(pin_f32(w.o[d][4 * j] * inv), pin_f32(w.o[d][4 * j + 1] * inv));
+      x.y = pack2<BF16>(pin_f32(w.o[d][4 * j + 2] * inv), pin_f32(w.o[d][4 * j + 3] * inv));
+      *(uint2v*)(op + (pK > 0 ? (2 * d + (j >> 1)) * 512 + (j & 1) * 256 : 32 * d + 8 * j)) = x;
+    }
+}
+
+// Where a block works: the query tiles of one (b, h) read the same K / V rows,
+// so they are consecutive blocks of one XCD's share (blocks are dealt to the 8
+// XCDs in turn) and share its L2; the (b, h) pairs are dealt to the XCDs in
+// turn, which spreads sequences of different lengths, or, without a multiple
+// of 8 pairs, in contiguous runs.
+__device__ __forceinline__ void sdpa_block(int nqt, int nh, int& qt, int& b, int& h) {
+  const int nbh = (int)(gridDim.x / nqt);
+  int bh;
+  if ((nbh & 7) == 0) {
+    const int x = blockIdx.x & 7, idx = blockIdx.x >> 3;
+    qt = idx % nqt;
+    bh = (idx / nqt) * 8 + x;
+  } else {
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    qt = t % nqt;
+    bh = t / nqt;
+  }
+  h = bh % nh;
+  b = bh / nh;
+}
+
+// Classes of up to 64 key tiles: lane i gets the class of tile base + i for the
+// wave's own 32 queries qw .. (0 skip, 1 all visible, 2 mixed) in *mine;
+// returns the tiles some wave of the block (NW waves, queries q0 ..) needs.
+template <int NW>
+__device__ __forceinline__ uint64_t tile_classes(const uint8_t* cls, const uint8_t* mask, int b, int q0, int wave, int Lq,
+                                                 int Lk, int nkt, int base, int lane, uint32_t* mine) {
+  const int kt = base + lane, qw = q0 + 32 * wave;
+  uint32_t any = 0, c = 0;
+  if (kt < nkt) {
+    if (cls != nullptr) {
+      const int nqt128 = (Lq + kBQ - 1) / kBQ;
+#pragma unroll
+      for (int i = 0; i < NW; i++) {
+        const int qq = q0 + 32 * i;
+        if (qq >= Lq) break;
+        const uint32_t x =
+            *(const uint16_t*)(cls + (((int64_t)b * nqt128 + qq / kBQ) * nkt + kt) * kNW + ((qq >> 4) & 7));
+        any |= x;
+        if (i == wave) c = x;
+      }
+      const uint32_t c0 = c & 255u, c1 = qw + 16 < Lq ? c >> 8 : c0;  // (groups past Lq have class 0)
+      c = c0 == c1 ? c0 : 2u;
+    } else {
+      c = qw >= Lq ? 0u : mask == nullptr && (kt + 1) * kBK <= Lk ? 1u : 2u;
+      any = 1;
+    }
+  }
+  *mine = c;
+  return __ballot(any != 0);
+}
+
+// A K or V tile by direct-to-LDS loads: 8 pieces of 1 KB (8 rows); a piece's
+// lane l fills slot l % 8 of row l / 8, so it fetches chunk (l % 8) ^
+// kv_f(row).  Rows past Lk become zeros.
+__device__ __forceinline__ void dma_piece(const uint16_t* base, int64_t stride, int k0, int piece, int Lk, uint16_t* dst,
+                                          int lane) {
+  const uint64_t a = (uint64_t)(base + (int64_t)k0 * stride);
+  const uint4v rs = {(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a),
+                     (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu), 0x80000000u, 0x00020000u};
+  const int r = piece * 8 + (lane >> 3);
+  const uint32_t off = __umul24(r, (uint32_t)stride) * 2u + (((lane & 7) ^ kv_f(r)) << 4);
+  const uint32_t lds = (uint32_t)__builtin_amdgcn_readfirstlane(
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)(dst + piece * 512));
+  buffer_to_lds16(rs, k0 + r < Lk ? off : 0xfffffff0u, lds);
+}
+
+struct KPair {  // a K row's chunks c and c + 4 and their rotation
+  uint4v lo, hi;
+  float2 cs[8];
+};
+// (rows past Lk repeat the last one: their scores are hidden)
+__device__ __forceinline__ void kpair_load(KPair& p, const uint16_t* Kb, int64_t stride, const float2* tab, int k0, int r,
+                                           int c, int Lk) {
+  const int rr = k0 + r < Lk ? r : Lk - 1 - k0;
+  load_pair(Kb + (int64_t)k0 * stride + __umul24(rr, (uint32_t)stride), true, c, p.lo, p.hi);
+  load_cs(tab + (int64_t)k0 * 32, rr, c, p.cs);
+}
+template <bool BF16>
+__device__ __forceinline__ void kpair_store(KPair& p, uint16_t* tile, int r, int c) {
+  rot_pair<BF16>(p.lo, p.hi, p.cs);
+  *(uint4v*)(tile + r * 64 + ((c ^ kv_f(r)) << 3)) = p.lo;
+  *(uint4v*)(tile + r * 64 + (((c + 4) ^ kv_f(r)) << 3)) = p.hi;
+}
+
+// K and V tiles in a two-buffer LDS ring, one barrier per tile, four waves of
+// 32 queries.  What bounds it: a wave's tile is ~200 VALU instructions (32 exp2,
+// fma, add and 16 packed conversions of scores among them) and 16 MFMAs; at
+// T = 2048 the SIMDs issue VALU 58% and MFMA 30% of the time, and the two
+// overlap little.  Against the 16-query kernel a staged tile and its fragment
+// reads serve twice the queries, and nothing of V passes through registers.
+// Three blocks per CU (168 VGPRs); four, at 128 VGPRs, measured the same, eight
+// waves a block slower (T 512 B 32 50 -> 58 us).  T = 2048, B = 16, 16 heads:
+// 566 -> 434 us (635 TFLOP/s), T = 8192, B = 1, 12 heads 460 -> 322 us.
+template <bool BF16, int NW, bool ROPEK>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(3))) void sdpa32_ring(
+    const uint16_t* __restrict__ Q, S4 qs, const uint16_t* __restrict__ K, S4 ks, const uint16_t* __restrict__ V, S4 vs,
+    const uint8_t* __restrict__ mask, S4 ms, int mask_vec, const uint8_t* __restrict__ cls, uint16_t* __restrict__ O,
+    S4 os, int Lq, int Lk, float scale_log2, const float2* __restrict__ tabq, const float2* __restrict__ tabk, int pK,
+    int nqt, int nh) {
+  static_assert(NW == 4, "K staging: one chunk pair per thread");
+  __shared__ __attribute__((aligned(16))) uint16_t Ks[2][kBK * 64];
+  __shared__ __attribute__((aligned(16))) uint16_t Vs[2][kBK * 64];
+  const int tid = threadIdx.x, lane = tid & 63, lg = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int qt, b, h;
+  sdpa_block(nqt, nh, qt, b, h);
+  const int q0 = qt * 32 * NW, q = q0 + 32 * wave + (lane & 31), qc = q < Lq ? q : Lq - 1;
+  const int nkt = (Lk + kBK - 1) / kBK;
+  const uint16_t* Kb = K + b * ks.s[0] + h * ks.s[1];
+  const uint16_t* Vb = V + b * vs.s[0] + h * vs.s[1];
+  const uint8_t* mrow = mask == nullptr ? nullptr : mask + b * ms.s[0] + (int64_t)qc * ms.s[2];
+
+  int base = 0;
+  uint32_t mine;
+  uint64_t need = tile_classes<NW>(cls, mask, b, q0, wave, Lq, Lk, nkt, 0, lane, &mine);
+  // the next tile some wave needs (nkt: none) and its class for this wave
+  auto next_tile = [&](uint32_t* c) -> int {
+    while (need == 0) {
+      base += 64;
+      if (base >= nkt) return nkt;
+      need = tile_classes<NW>(cls, mask, b, q0, wave, Lq, Lk, nkt, base, lane, &mine);
+    }
+    const int i = __builtin_ctzll(need);
+    need &= need - 1;
+    *c = (uint32_t)__builtin_amdgcn_readlane((int)mine, i);
+    return base + i;
+  };
+  Wave32 w;
+  wave32_init<BF16>(w, Q + b * qs.s[0] + h * qs.s[1] + (int64_t)qc * qs.s[2], tabq, qc, lg);
+
+  KPair kp;
+  const int kr = tid >> 2, kc = tid & 3;
+  auto fetch = [&](int kt, int bf) __attribute__((always_inline)) {
+    const int k0 = kt * kBK;
+#pragma unroll
+    for (int i = 0; i < 8 / NW; i++) dma_piece(Vb, vs.s[2], k0, wave * (8 / NW) + i, Lk, Vs[bf], lane);
+    if constexpr (ROPEK) {
+      kpair_load(kp, Kb, ks.s[2], tabk, k0, kr, kc, Lk);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8 / NW; i++) dma_piece(Kb, ks.s[2], k0, wave * (8 / NW) + i, Lk, Ks[bf], lane);
+    }
+  };
+  // everything requested has landed (before the barrier that publishes it)
+  auto landed = [&](int bf) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (ROPEK) kpair_store<BF16>(kp, Ks[bf], kr, kc);
+  };
+  uint32_t cl = 0;
+  int kt = next_tile(&cl), bf = 0;
+  if (kt < nkt) {
+    fetch(kt, 0);
+    landed(0);
+  }
+  const Frag32 f = frag32(lane);
+  __syncthreads();
+  while (kt < nkt) {
+    // the next tile into the other buffer (free since the last barrier)
+    uint32_t ncl = 0;
+    const int nk = next_tile(&ncl);
+    if (nk < nkt) fetch(nk, bf ^ 1);
+    if (cl != 0)
+      wave32_tile<BF16>(w, f, Ks[bf], Vs[bf], kt * kBK, Lk, cl == 2, mrow, ms.s[3], mask_vec, scale_log2, lg);
+    if (nk < nkt) landed(bf ^ 1);
+    kt = nk;
+    cl = ncl;
+    bf ^= 1;
+    __syncthreads();
+  }
+  wave32_store<BF16>(w, O, os, pK, b, h, q, Lq, lg);
 }
 
 // ------------------------------------------------------------------ f32 MFMA kernel (D = 64)
@@ -1013,7 +1434,6 @@ static void sdpa_impl(uintptr_t ctx, int dt, uintptr_t q, const int64_t* qs, uin
     int nqt = (int)((Lq + kBQ - 1) / kBQ);
     uint8_t* info = (uint8_t*)mask_info;
     uint8_t* tmp = nullptr;
-    int mask_vec = 0;
     if (mask) {
       if (!info) {
         HB_REQUIRE(!noalloc, "hb_sdpa_noalloc: no mask summary");
@@ -1022,22 +1442,61 @@ static void sdpa_impl(uintptr_t ctx, int dt, uintptr_t q, const int64_t* qs, uin
         check_launch("hb_sdpa(mask info)");
         info = tmp;
       }
-      mask_vec = ms[3] == 1 && mask % 8 == 0 && ms[0] % 8 == 0 && ms[2] % 8 == 0;
     } else {
       info = nullptr;
     }
     const float sl2 = scale * 1.4426950408889634f;
     const int64_t nblk = (int64_t)nqt * H * B;
     HB_REQUIRE(nblk < ((int64_t)1 << 31), "hb_sdpa: too many (batch, head, query tile) blocks");
-    const unsigned grid = (unsigned)nblk;
-    if (dt == HB_F16)
-      sdpa_mfma<false><<<grid, kNT, 0, st>>>((const uint16_t*)q, Qs, (const uint16_t*)k, Ks, (const uint16_t*)v, Vs,
-                                             (const uint8_t*)mask, Ms, mask_vec, info, (uint16_t*)o, Os, (int)Lq,
-                                             (int)Lk, sl2, tq, tk, pK, nqt, (int)H);
-    else
-      sdpa_mfma<true><<<grid, kNT, 0, st>>>((const uint16_t*)q, Qs, (const uint16_t*)k, Ks, (const uint16_t*)v, Vs,
-                                            (const uint8_t*)mask, Ms, mask_vec, info, (uint16_t*)o, Os, (int)Lq,
-                                            (int)Lk, sl2, tq, tk, pK, nqt, (int)H);
+    // Which kernel: by the shape and the kind of mask only, never by the number
+    // of sequences, so that a sequence's bits do not depend on its batch.  The
+    // 32-query kernel wins where every query reads every key, or the
+    // sequence is long (its blocks are fewer and do more per tile); with a
+    // windowed mask on up to 1024 keys the 16-query one has the shorter chain
+    // per block.  us, 16 / 32 queries a wave, 12 heads (16 from T = 1024),
+    // padded below T = 1024, RoPE on both operands:
+    //   every key:  T 128 B 1 9.0 / 9.6, T 384 B 8 18.9 / 19.3, T 512 B 4 19.0 /
+    //               18.3, T 512 B 32 55.4 / 50.2, T 2048 B 16 566 / 465
+    //   windowed:   T 512 B 8 23.4 / 26.3, T 512 B 32 53.0 / 53.2, T 1024 B 8
+    //               59.1 / 61.3, T 2048 B 16 125 / 121
+    const bool all_keys = !mask || ms[2] == 0;
+    const bool wide = Lk > 1024 || (all_keys && Lk > 384);
+    if (wide) {
+      // From 1024 keys that every query tile reads, K is rotated once in a pass
+      // of its own instead of by every block that stages it (T 2048 B 16 465 ->
+      // 434, T 8192 B 1 367 -> 322 us, the pass included; T 512 B 32 50 -> 54).
+      struct PoolBlock {  // back to the pool when the call ends, by return or throw
+        uintptr_t ctx;
+        void* p;
+        ~PoolBlock() {
+          if (p) pool_free(ctx, p);  // stream-ordered: reused only by work enqueued later
+        }
+      } rotated{ctx, nullptr};
+      const int64_t kblk = (Lk + 63) / 64 * B * H;
+      if (tk && all_keys && Lk >= 1024 && kblk < ((int64_t)1 << 31)) {
+        rotated.p = pool_alloc(ctx, (size_t)(B * H * Lk * 64 * 2));
+        auto kern = dt == HB_F16 ? rope_k_kernel<false> : rope_k_kernel<true>;
+        kern<<<(unsigned)kblk, 256, 0, st>>>((const uint16_t*)k, Ks, (uint16_t*)rotated.p, (int)Lk, (int)H, (int)(B * H),
+                                             tk);
+        check_launch("hb_sdpa (rotate K)");
+        k = (uintptr_t)rotated.p;
+        Ks = S4{{H * Lk * 64, Lk * 64, 64, 1}};
+        tk = nullptr;
+      }
+      const int mask_vec = mask && ms[3] == 1 && mask % 16 == 0 && ms[0] % 16 == 0 && ms[2] % 16 == 0;
+      auto kern = dt == HB_F16 ? (tk ? sdpa32_ring<false, 4, true> : sdpa32_ring<false, 4, false>)
+                               : (tk ? sdpa32_ring<true, 4, true> : sdpa32_ring<true, 4, false>);
+      kern<<<(unsigned)nblk, 256, 0, st>>>((const uint16_t*)q, Qs, (const uint16_t*)k, Ks, (const uint16_t*)v, Vs,
+                                           (const uint8_t*)mask, Ms, mask_vec, info, (uint16_t*)o, Os, (int)Lq, (int)Lk,
+                                           sl2, tq, tk, pK, nqt, (int)H);
+    } else {
+      // 8 contiguous mask bytes per lane and load, of any alignment
+      const int mask_vec = mask && ms[3] == 1;
+      auto kern = dt == HB_F16 ? sdpa_mfma<false> : sdpa_mfma<true>;
+      kern<<<(unsigned)nblk, kNT, 0, st>>>((const uint16_t*)q, Qs, (const uint16_t*)k, Ks, (const uint16_t*)v, Vs,
+                                           (const uint8_t*)mask, Ms, mask_vec, info, (uint16_t*)o, Os, (int)Lq, (int)Lk,
+                                           sl2, tq, tk, pK, nqt, (int)H);
+    }
     check_launch("hb_sdpa");
     if (tmp) pool_free(ctx, tmp);
   } else if (sdpa_takes_f32(dt, q, qs, k, ks, v, vs, o, os, Lk, D)) {
