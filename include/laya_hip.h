@@ -183,10 +183,9 @@ int hb_graph_destroy(uintptr_t ctx, uintptr_t exec);
 int hb_linear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintptr_t w, uintptr_t bias, uintptr_t resid,
               int64_t ldr, uintptr_t y, int64_t ldy, int64_t M, int64_t N, int64_t K, unsigned flags);
 /*  HB_X_PANEL / HB_Y_PANEL (hb_linear and hb_qlinear): x read from / y
- *  written in panel order.  Taken by two kernels: dt f16 or bf16,
- *  K % 64 == 0, 16-byte aligned operands, and either M >= 4096 (the large-M
- *  kernel), or, for hb_linear only, a call that takes the small-M slab
- *  kernel: 64 * K * (2 with GeGLU) <= 160 KiB and
+ *  written in panel order.  Taken for dt f16 or bf16, K % 64 == 0, 16-byte
+ *  aligned operands, and either M >= 4096, or, for hb_linear only, a small
+ *  call: 64 * K * (2 with GeGLU) <= 160 KiB and
  *  ceil(N / 32) * ceil(M / 128) <= the device's CUs (hb_device_info "cus").
  *  A panel-order y also needs N % 16 == 0 and no residual.  Other calls
  *  fail.  The arithmetic is the same as with row-major operands, bit for
@@ -215,10 +214,9 @@ int hb_linear_qkv(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintptr_t w, 
  * `zeros` are f16 [N, ceil(K/group)].  Weights dequantize to
  * fl16(q*s + z) (fl16(q*s) when symmetric), exactly what host
  * dequantization uploads, and feed the f16 MFMA with f32 accumulation
- * (M >= 4096, and M >= 1024 for calls that neither the small-M slab
- * kernel nor 128 x 64 tiles take: once per call into a 16-bit copy taken
- * from the context's pool for the duration of the call; otherwise inside
- * the GEMM kernels' weight loaders).
+ * (K % 64 == 0 or M >= 4096, and large calls below that: once per call into
+ * a 16-bit copy taken from the context's pool for the duration of the call;
+ * otherwise inside the GEMM kernel's weight loader).
  * Backend.quantizedLinear (index.ts:257-261) via compose.quantizedLinear
  * (compose.ts:407-414).
  *  dt     dtype of x / y / resid / bias: HB_F16, HB_BF16 or HB_F32.

@@ -11,9 +11,9 @@
 //   same LDS C tile) is staged in LDS and written during the first stages of
 //   the block's next tile.  X and Y may be row-major or in panel order
 //   (32-row x 16-column blocks of 1 KB laid out as MFMA operands);
-// - gemm_slab (small M, K % 64 == 0): weight-stationary, the whole W slab of
-//   a block in LDS, every X fragment in registers, one wait for memory;
-// - gemm_mfma (the rest below M = 4096): 128 x 128 tiles, A and B
+// - gemm_ring (K % 64 == 0, smaller M): X and W through an LDS ring of K stages
+//   filled by direct loads, one barrier per stage; row-major or panel order;
+// - gemm_mfma (other K below M = 4096): 128 x 128 or 128 x 64 tiles, A and B
 //   double-buffered in LDS, epilogue staged in LDS, 16-byte stores.
 // W tiles are 64-wide K stages of 16-byte chunks XOR-swizzled by row so the
 // fragment reads of consecutive rows spread over the LDS banks.  The
@@ -22,9 +22,8 @@
 // (y = round(round(x.w^T + b) + r), the linear-then-add order).  Quantized
 // weights are dequantized to fl16(q*s + z) -- one correctly rounded f16 fma,
 // the value host dequantization would upload -- by one routine (dequant8):
-// in the 128 x 128 kernel's W loader, into the slab in LDS, and from
-// M = 1024 on (unless the slab kernel takes the call) once per call into a
-// pooled 16-bit copy that the 16-bit kernels then read (dequant_rows_kernel).
+// once per call into a pooled 16-bit copy that the 16-bit kernels then read
+// (dequant_rows_kernel), or in gemm_mfma's W loader.
 // Blocks walk the tile grid in an XCD-aware order: the hardware deals block b
 // to XCD b % 8, so each XCD is given a contiguous run of row panels (their A
 // rows and the whole W stay in that XCD's L2).
@@ -170,15 +169,15 @@ static bool dot_shape(int64_t M, int64_t N, int64_t K) { return M * N <= 16384 &
 
 // Panel-order operands (HB_X_PANEL / HB_Y_PANEL) need K % 64 == 0 and one of
 // the two kernels that take them: the large-M one (M >= 4096) or, for 16-bit
-// weights, the small-M slab kernel (`slab`: the call takes it); a panel-order
+// weights, the calls of small_panel_path (`small`); a panel-order
 // Y also a width of whole 16-column blocks and no residual.
-static void check_panel(unsigned flags, bool mfma, bool slab, int64_t M, int64_t N_out, int64_t K, bool resid,
+static void check_panel(unsigned flags, bool mfma, bool small, int64_t M, int64_t N_out, int64_t K, bool resid,
                         const char* op) {
   if (!(flags & (HB_X_PANEL | HB_Y_PANEL))) return;
-  if (!mfma || !(arow_path(M) || slab) || K % 64 != 0)
+  if (!mfma || !(arow_path(M) || small) || K % 64 != 0)
     throw std::runtime_error(std::string(op) +
                              ": panel-order operands need f16/bf16, K % 64 == 0, 16-byte aligned operands and "
-                             "M >= 4096, or (16-bit weights) the small-M slab kernel");
+                             "M >= 4096, or (16-bit weights) one of the small calls that take them");
   if ((flags & HB_Y_PANEL) && (N_out % 16 != 0 || resid))
     throw std::runtime_error(std::string(op) + ": a panel-order y needs out % 16 == 0 and no residual");
 }
@@ -213,7 +212,7 @@ extern "C" int hb_linear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintpt
   hipStream_t st = stream_of(ctx);
   bool mfma = (dt == HB_F16 || dt == HB_BF16) && K > 0 && K % 8 == 0 && ldx % 8 == 0 && ldy % 8 == 0 &&
               (!r || ldr % 8 == 0) && x % 16 == 0 && w % 16 == 0 && y % 16 == 0 && (!r || resid % 16 == 0);
-  check_panel(flags, mfma, !arow_path(M) && slab_path(M, N, K, geglu, cu_count(ctx)), M, N, K, r != nullptr,
+  check_panel(flags, mfma, !arow_path(M) && small_panel_path(M, N, K, geglu, cu_count(ctx)), M, N, K, r != nullptr,
               "hb_linear");
   const unsigned pan = flags & (HB_X_PANEL | HB_Y_PANEL);
   if (mfma) {
@@ -331,16 +330,12 @@ extern "C" int hb_qlinear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintp
     uint16_t* Yp = (uint16_t*)y;
     int m = (int)M, n = (int)N, k = (int)K;
     const int cus0 = cu_count(ctx);
-    const bool slab = slab_path(M, N, K, geglu, cus0) && qslab_ok(K, geglu ? 2 : 1, bits, mode == 1, q);
-    if (arow_path(M) || (M >= 1024 && !slab && !thin_tiles(M, N, geglu, cus0))) {
-      // At M >= 4096, and from M = 1024 where neither the slab kernel nor
-      // 128 x 64 tiles take the call: the weight is dequantized once into a
-      // pooled 16-bit copy and the 16-bit GEMM runs on it.  A loader that
-      // dequantizes repeats the work for every row tile (at M = 8192:
-      // 22-34% over 16-bit weights, against one bandwidth-bound pass over
-      // the weight here).  With 128 x 64 tiles (many blocks, each a short
-      // chain of K stages) the loader's dequantization is the faster of the
-      // two (M = 2048: Wo 16.3 -> 14.6, Wqkv 27.9 -> 24.6 us).
+    if (arow_path(M) || ring_ok(ldx, K) || (M >= 1024 && !thin_tiles(M, N, geglu, cus0))) {
+      // The weight is dequantized once into a pooled 16-bit copy and the 16-bit
+      // GEMM runs on it: one bandwidth-bound pass over the weight (4-6 us)
+      // instead of the same work in every row tile's loader (M = 512, q4, the
+      // pass included: 1152 x 768 GeGLU 20.7 -> 12.5, 768 x 1152 18.8 -> 11 us).
+      // gemm_mfma dequantizes in its loader where it has few blocks.
       const int64_t rows = geglu ? 2 * N : N;
       struct PoolBlock {  // back to the pool when the call ends, by return or throw
         uintptr_t ctx;

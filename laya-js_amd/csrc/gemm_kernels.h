@@ -405,220 +405,250 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_mfma(const uint16_t* __restr
   write_tile<BF16, BM, BNO, NT>(Cs, m0, n0, M, N, R, ldr, Y, ldy);
 }
 
-// ------------------------------------------------------------------ small-M MFMA kernel
+// ------------------------------------------------------------------ ring MFMA kernel
 
-// Small-M GEMM for 16-bit weights (M < 4096, K % 64 == 0): weight-stationary,
-// one memory round trip.  A block of two or four waves owns a slab of
-// 32*TN W rows (the output columns n0 .. n0 + 32*TNO, and with GeGLU their
-// gate rows too) and one 32-row block of X per wave.  Everything a wave needs is
-// requested at once before anything is waited for: its X fragments for P k16
-// steps (P = K/16 when that fits in registers), its residual and bias values,
-// and its share of the whole slab, which goes to LDS with direct-to-LDS loads
-// (global_load_lds: 16 bytes per lane, whole 128-byte lines of 8 rows per
-// instruction), so the kernel waits for memory once.  What bounds it is the
-// X fragment loads (32 rows x 32 bytes per 1 KB instruction), which a CU's L1
-// serves at about 15 bytes per clock; the launcher uses the kernel while its
-// blocks fit one per CU (Wqkv at M = 128: 72 blocks, 11 us against 15 us for
-// the 128 x 128 kernel, which ran 18 blocks).
-// The k16 steps then run in ascending order with the same MFMA, operand
-// order (W rows as the A operand, X rows as the B operand) and epilogue as
-// the other kernels, so a row's bits do not depend on M.
-// Slab layout: 1 KB blocks of 8 rows x 64 k, block (r/8)*KB + k/64 (KB = K/64),
-// 16-byte chunk c of row r at slot (r%8)*8 + (c ^ (r%8)), so the 8 lanes of a
-// fragment read that share a row group hit 8 distinct bank groups.  Blocks
-// are numbered row-chunk-fastest and dealt to XCDs in contiguous runs: the
-// blocks that read one slab share an XCD's L2.
-//
-// Quantized weights (QB = 8 or 4, f16 scales and zeros, groups a multiple of
-// 8): the slab's codes (its rows are contiguous runs of the code matrix) and
-// its scales and zeros go to LDS by direct-to-LDS loads beside the f16 slab,
-// and after the one wait every thread dequantizes its share of the slab's
-// 8-weight chunks into the f16 slab (dequant8, the other kernels' rounding),
-// so the MFMA steps and their bits are those of the 16-bit path.
-template <int TN, int P, bool BF16, bool GEGLU, int QB = 0, bool AFF = false>
-__global__ __launch_bounds__(256) void gemm_slab(const uint16_t* __restrict__ X, int64_t ldx,
-                                                 const uint16_t* __restrict__ W, QW qw,
-                                                 const uint16_t* __restrict__ bias,
-                                                 const uint16_t* __restrict__ R, int64_t ldr, uint16_t* __restrict__ Y,
-                                                 int64_t ldy, int M, int N, int K, int chunks, int xpan, int ypan) {
-  constexpr int TNO = GEGLU ? TN / 2 : TN;  // output column blocks
-  constexpr int SR = 32 * TN;               // slab rows
-  static_assert(!GEGLU || TN % 2 == 0, "GEGLU needs value and gate blocks");
-  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, lg = lane >> 5;
-  const int nw = blockDim.x >> 6;  // waves per block (2 or 4): 32 rows of X each
-  const int t = xcd_tile(blockIdx.x, gridDim.x);
-  const int nt = t / chunks, mc = t - nt * chunks;
-  const int n0 = nt * 32 * TNO;
-  const int KB = K >> 6, S = K >> 4;  // 64-wide k blocks, k16 steps
-  const int row = (mc * nw + wave) * 32 + l32;  // this lane's output row
-  // X row-major, or in panel order (xpan: 32-row x 16-column blocks of 1 KB
-  // in MFMA operand order, rows padded to a multiple of 32), where one
-  // fragment load reads one whole block; rows past the operand are clamped
-  const int mlim = xpan ? (M + 31) & ~31 : M, rc = row < mlim ? row : mlim - 1;
-  const int64_t xoff = xpan ? (int64_t)(rc >> 5) * 32 * K + (rc & 31) * 8 + 256 * lg : (int64_t)rc * ldx + 8 * lg;
-  const int xstep = xpan ? 512 : 16;  // elements per k16 step
+// GEMM for 16-bit weights and K % 64 == 0, from one row up to where the large-M
+// kernel's tiles fill the chip.  Both operands go to an LDS ring of NST 64-wide K
+// stages by direct loads (no registers, so requests run stages ahead whatever the
+// wave is doing), with one barrier per stage; waves of 32 x 32 outputs (32 x 64 in
+// the widest tile) read each k16 step's fragments one step ahead.
+// What bounds it: up to one 64 x 64 tile per CU the chain of K stages, 0.17 us
+// each (four waves share the ring's requests and fragment reads: two took 0.26),
+// behind about 4 us of launch, first load and write-out; at several tiles per CU
+// LDS, which a wave of 32 x 32 reads 2 KB of per 32-clock MFMA.  The kernels
+// before it waited for each stage's loads (gemm_mfma: 0.8 us a stage) or loaded X
+// fragments of 32 rows x 32 bytes from global memory (a slab kernel).  Measured
+// (us, f16, before -> after): 128 x 2304 x 768 9.3 -> 5.6, 128 x 2304 x 768 GeGLU
+// 15.1 -> 5.9, 128 x 768 x 3072 32.7 -> 11.3, 2048 x 768 x 1152 15.6 -> 9.1, 2048
+// x 2304 x 768 21.9 -> 17.6 (413 TFLOP/s).
+// Same MFMA, operand order (W rows as the A operand, X rows as the B operand) and
+// ascending k16 steps as the other kernels: a row's bits do not depend on M or on
+// the tile.
+// 16 bytes per lane from buffer `rs` at byte offsets voff + soff straight into
+// LDS [lds + 16 lane, + 16).  Inline asm: the compiler neither holds LDS reads
+// behind it nor counts it in its waits; the caller waits (vmcnt).
+__device__ __forceinline__ void ring_dma16(const uint4v& rs, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rs), "s"(soff),
+               "s"(lds)
+               : "memory");
+}
+template <int N>
+__device__ __forceinline__ void ring_wait_barrier() {
+  // this wave's loads up to the stage about to be read have landed, its LDS
+  // reads of the last stage are done; then everybody's
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
 
-  uint4v xf[P];
-#pragma unroll
-  for (int p = 0; p < P; p++) xf[p] = *(const uint4v*)(X + xoff + xstep * p);
-  // epilogue inputs: the residual and the bias of the lane's 4-column groups
-  // (8-byte loads where aligned: R rows are, ldr % 8 == 0; the bias may be a
-  // view at any offset, and its gate half starts at N)
-  const bool bvec = bias != nullptr && ((uintptr_t)bias & 7) == 0 && (!GEGLU || (N & 3) == 0);
-  uint2v rres[TNO][4], rb[TNO][4], rbg[TNO][4];
-#pragma unroll
-  for (int j = 0; j < TNO; j++)
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-      const int col = n0 + 32 * j + 8 * g + 4 * lg;
-      const bool whole = row < M && col + 4 <= N;
-      rres[j][g] = R != nullptr && whole ? *(const uint2v*)(R + (int64_t)row * ldr + col) : uint2v{0, 0};
-      rb[j][g] = bvec && col + 4 <= N ? *(const uint2v*)(bias + col) : uint2v{0, 0};
-      rbg[j][g] = GEGLU && bvec && col + 4 <= N ? *(const uint2v*)(bias + N + col) : uint2v{0, 0};
-    }
-  // slab row r -> W row (GeGLU: gate rows from SR / 2 on); rows past N are
-  // clamped, their outputs never stored
-  auto slab_wrow = [&](int r) -> int {
-    const bool gate = GEGLU && r >= SR / 2;
-    const int cc = n0 + (gate ? r - SR / 2 : r);
-    return (cc < N ? cc : N - 1) + (gate ? N : 0);
-  };
-  const int nq = (SR / 8) * KB;
-  // quantized: codes [SR][K * QB / 8 bytes], then scales and zeros [SR][G],
-  // each f16 in the low half of a 32-bit slot (a 2-byte direct-to-LDS load
-  // writes lane l's value at 4 l), after the f16 slab
-  constexpr int CRB = QB ? 8 / QB : 1;  // weights per code byte (QB = 4: 2)
-  const int rowb = QB ? K / CRB : 0;     // code bytes per row
-  uint8_t* codes = (uint8_t*)(smem + SR * K);
-  uint32_t* szs = (uint32_t*)(codes + SR * rowb);
-  if constexpr (QB == 0) {
-    // the slab: DMA instruction q (of wave q % nw) fills block q, i.e. slab
-    // rows 8 * (q / KB) + lane / 8, k block q % KB; lane l fetches chunk
-    // (l%8) ^ (row%8)
-    for (int q = wave; q < nq; q += nw) {
-      const int rb8 = q / KB, kb = q - rb8 * KB;
-      const int r = rb8 * 8 + (lane >> 3), c = (lane & 7) ^ (r & 7);
-      __builtin_amdgcn_global_load_lds((const void*)(W + (int64_t)slab_wrow(r) * K + kb * 64 + c * 8),
-                                       (__attribute__((address_space(3))) void*)(smem + q * 512), 16, 0, 0);
-    }
+// ... with at most `later` (up to MOST) stages of PW loads each still in flight
+template <int PW, int MOST>
+__device__ __forceinline__ void ring_wait_stages(int later) {
+  if constexpr (MOST <= 0) {
+    ring_wait_barrier<0>();
   } else {
-    // codes: instruction q fills bytes [1024 q, 1024 q + 1024) of the code
-    // block, 16 of one row per lane (rowb % 16 == 0)
-    const int ncq = SR * rowb / 1024;
-    for (int q = wave; q < ncq; q += nw) {
-      const int b = q * 1024 + lane * 16, r = b / rowb;
-      __builtin_amdgcn_global_load_lds((const void*)(qw.q + (int64_t)slab_wrow(r) * rowb + (b - r * rowb)),
-                                       (__attribute__((address_space(3))) void*)(codes + q * 1024), 16, 0, 0);
-    }
-    // scales (then zeros): 2 bytes per lane into 4-byte slots, instruction q
-    // entries [64 q, 64 q + 64) of the slab's [SR][G]
-    const int G = qw.G, nsq = (SR * G + 63) / 64;
-    for (int q = wave; q < (AFF ? 2 : 1) * nsq; q += nw) {
-      const bool zq = q >= nsq;
-      const int e = (zq ? q - nsq : q) * 64 + lane, r = e / G;
-      if (e < SR * G)
-        __builtin_amdgcn_global_load_lds(
-            (const void*)((const uint16_t*)(zq ? qw.zeros : qw.scales) + (int64_t)slab_wrow(r) * G + (e - r * G)),
-            (__attribute__((address_space(3))) void*)(szs + (zq ? SR * G : 0) + (q - (zq ? nsq : 0)) * 64), 2, 0,
-            0);
-    }
+    if (later >= MOST) ring_wait_barrier<MOST * PW>();
+    else ring_wait_stages<PW, MOST - 1>(later);
   }
-  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0): everything above has landed
-  __syncthreads();
-  if constexpr (QB != 0) {
-    // dequantize: chunk i (8 weights) is slab row i / (K/8), chunk i % (K/8)
-    // of the row, into the f16 slab's layout
-    const int cpr = K >> 3, G = qw.G, nth = nw * 64;
-    for (int i = tid; i < SR * cpr; i += nth) {
-      const int r = i / cpr, c = i - r * cpr;
-      uint32_t w0, w1 = 0;
-      if constexpr (QB == 8) {
-        const uint2v w = *(const uint2v*)(codes + r * rowb + 8 * c);
-        w0 = w.x;
-        w1 = w.y;
+}
+
+template <int BM, int BN, int WM, int WN, int NST, bool BF16, bool GEGLU>
+__global__ __launch_bounds__(WM* WN * 64) void gemm_ring(const uint16_t* __restrict__ X, int64_t ldx,
+                                                         const uint16_t* __restrict__ W,
+                                                         const uint16_t* __restrict__ bias,
+                                                         const uint16_t* __restrict__ R, int64_t ldr,
+                                                         uint16_t* __restrict__ Y, int64_t ldy, int M, int N, int K,
+                                                         int tiles_n, int xpan, int ypan) {
+  constexpr int NW = WM * WN, NT = NW * 64;
+  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
+  constexpr int PCS = (BM + BN) / 8, PW = PCS / NW;  // 1 KB pieces (8 rows x 64 k) per stage, per wave
+  constexpr int STAGE = (BM + BN) * 64;              // u16 per stage
+  constexpr int BNO = GEGLU ? BN / 2 : BN;
+  static_assert(PW * NW == PCS, "whole rounds of pieces");
+  static_assert(!GEGLU || (BN / 2) % 32 == 0, "value blocks, then gate blocks");
+  static_assert(NST >= 3, "a stage is published one stage ahead");
+  static_assert(PW * (NST - 2) <= 63, "vmcnt immediate");
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lg = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int m0 = (tile / tiles_n) * BM, n0 = (tile % tiles_n) * BNO;
+
+  // A stage is 1 KB pieces: X rows, then W rows (GeGLU: value rows, then gate
+  // rows).  Row-major piece p is tile rows 8 p .. 8 p + 7: lane l fills slot
+  // l % 8 of row l / 8, so it fetches chunk (l % 8) ^ f(row), f(r) = (r / 2) % 8,
+  // and the 16 lanes of a fragment-read pass (16 rows, one chunk) cover all 64
+  // banks.  With X in panel order (xpan) piece p is k16 block p % 4 of 32-row
+  // group p / 4, already a fragment.  Rows past the operand are clamped (their
+  // outputs are never stored).
+  const uint64_t xa = (uint64_t)(xpan ? X + (int64_t)(m0 >> 5) * 32 * K : X + (int64_t)m0 * ldx);
+  uint32_t off[PW], step[PW];  // byte offsets of the lane's 16 bytes, and per stage
+  uint4v rsrc[PW];             // W: the base is the piece's first row
+#pragma unroll
+  for (int i = 0; i < PW; i++) {
+    const int p = wave * PW + i, r = p * 8 + (lane >> 3);
+    const uint32_t c = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+    uint64_t base;
+    step[i] = 128;
+    if (p * 8 < BM) {
+      base = xa;
+      if (xpan) {
+        const int last = ((M + 31) >> 5) - 1 - (m0 >> 5), grp = min(p >> 2, last);
+        off[i] = (uint32_t)grp * (uint32_t)K * 64u + (uint32_t)(p & 3) * 1024u + (uint32_t)lane * 16u;
+        step[i] = 4096;
       } else {
-        w0 = *(const uint32_t*)(codes + r * rowb + 4 * c);
+        off[i] = (uint32_t)(m0 + r < M ? r : M - 1 - m0) * (uint32_t)ldx * 2u + c;
       }
-      const int gi = r * G + (8 * c) / qw.group;
-      const uint32_t sb = szs[gi] & 0xffffu, zb = AFF ? szs[SR * G + gi] & 0xffffu : 0u;
-      *(uint4v*)(smem + ((r >> 3) * KB + (c >> 3)) * 512 + (r & 7) * 64 + (((c & 7) ^ (r & 7)) << 3)) =
-          dequant8<QB, AFF, false, BF16>(w0, w1, sb, zb, 0.f, 0.f);
+    } else {
+      const int wr = r - BM, wr0 = p * 8 - BM;  // (a piece never straddles the halves)
+      const bool gate = GEGLU && wr0 >= BN / 2;
+      const int n = n0 + (gate ? wr - BN / 2 : wr), nb = n0 + (gate ? wr0 - BN / 2 : wr0);
+      const int nc = n < N ? n : N - 1, nbc = nb < N ? nb : N - 1;
+      base = (uint64_t)(W + (int64_t)(nbc + (gate ? N : 0)) * K);
+      off[i] = (uint32_t)(nc - nbc) * (uint32_t)K * 2u + c;
     }
-    __syncthreads();
+    rsrc[i] = uint4v{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base),
+                     (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32) & 0xffffu), 0x80000000u, 0x00020000u};
   }
-  if ((mc * nw + wave) * 32 >= M) return;  // a wave past the last row (after the barriers: its share is done)
-
-  // W fragment of column block j, k16 step s (slab row 32 j + l32)
-  auto wfrag = [&](int j, int s) __attribute__((always_inline)) -> uint4v {
-    const int r = 32 * j + l32, c = (2 * s + lg) & 7;
-    return *(const uint4v*)(smem + ((r >> 3) * KB + (s >> 2)) * 512 + (r & 7) * 64 + ((c ^ (r & 7)) << 3));
+  const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane(
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)smem);
+  auto issue = [&](int kt, int slot, int i0, int i1) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = i0; i < i1; i++)
+      ring_dma16(rsrc[i], off[i], (uint32_t)kt * step[i], lds0 + (uint32_t)(slot * STAGE * 2 + (wave * PW + i) * 1024));
   };
-  float16v acc[TN];
+
+  float16v acc[TM][TN];
 #pragma unroll
-  for (int j = 0; j < TN; j++)
+  for (int i = 0; i < TM; i++)
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[j][e] = 0.f;
-  for (int s0 = 0; s0 < S; s0 += P) {  // S % P == 0
+    for (int j = 0; j < TN; j++)
 #pragma unroll
-    for (int p = 0; p < P; p++) {
-      uint4v b[TN];
+      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+  // fragment chunk 2 s + lg of row l32 (f depends on l32 alone: blocks start at multiples of 32 rows)
+  int fo[4];
 #pragma unroll
-      for (int j = 0; j < TN; j++) b[j] = wfrag(j, s0 + p);
+  for (int s = 0; s < 4; s++) fo[s] = l32 * 64 + (((2 * s + lg) ^ ((l32 >> 1) & 7)) << 3);
+  int xo[4];  // X's, the same unless it is in panel order
 #pragma unroll
-      for (int j = 0; j < TN; j++) acc[j] = mfma32<BF16>(b[j], xf[p], acc[j]);
-      if (s0 + P < S) xf[p] = *(const uint4v*)(X + xoff + xstep * (s0 + P + p));  // K longer than the registers
+  for (int s = 0; s < 4; s++) xo[s] = xpan ? s * 512 + lane * 8 : fo[s];
+  // Fragments of a k16 step are read one step ahead of its MFMAs, across stages
+  // too: a stage is published one stage before it is multiplied.
+  uint4v xf[2][TM], wf[2][TN];
+  auto read = [&](int slot, int s, int d) __attribute__((always_inline)) {
+    const uint16_t* b = smem + slot * STAGE;
+#pragma unroll
+    for (int i = 0; i < TM; i++) xf[d][i] = *(const uint4v*)(b + xo[s] + (wm * WTM + i * 32) * 64);
+#pragma unroll
+    for (int j = 0; j < TN; j++) wf[d][j] = *(const uint4v*)(b + fo[s] + (BM + wn * WTN + j * 32) * 64);
+  };
+  // req >= 0: stage `req` is requested into slot `rs` between the MFMAs
+  auto compute = [&](int slot, int next, bool more, int req, int rs) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {  // k16 steps in order, W rows as A, X rows as B: the other kernels' bits
+      if (s < 3) read(slot, s + 1, (s + 1) & 1);
+      else if (more) read(next, 0, 0);
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = mfma32<BF16>(wf[s & 1][j], xf[s & 1][i], acc[i][j]);
+      if (req >= 0) issue(req, rs, s * PW / 4, (s + 1) * PW / 4);
+    }
+  };
+
+  const int KT = K >> 6;
+  // stages 0 .. NST - 2 in flight; stage 0 landed
+#pragma unroll
+  for (int s = 0; s < NST - 1; s++)
+    if (s < KT) issue(s, s, 0, PW);
+  ring_wait_stages<PW, NST - 2>(KT - 1);
+  read(0, 0, 0);
+  int slot = 0, kt = 0;
+  auto succ = [](int v) { return v == NST - 1 ? 0 : v + 1; };
+  // stage kt: stage kt + 1 has landed and everybody is done with stage kt - 1,
+  // whose slot takes stage kt + NST - 1
+  for (; kt + NST - 1 < KT; kt++) {
+    ring_wait_barrier<(NST - 3) * PW>();
+    compute(slot, succ(slot), true, kt + NST - 1, slot == 0 ? NST - 1 : slot - 1);
+    slot = succ(slot);
+  }
+  for (; kt < KT; kt++) {  // nothing more to request
+    ring_wait_stages<PW, NST - 3>(KT - 2 - kt);
+    compute(slot, succ(slot), kt + 1 < KT, -1, 0);
+    slot = succ(slot);
+  }
+  __syncthreads();
+
+  // ---- epilogue, as gemm_mfma's: bias, one rounding, staged in LDS as [BM][BN];
+  // GeGLU then pairs each value column with its gate on the way out
+  uint16_t* Cs = smem;
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+    const int orow = wm * WTM + i * 32 + l32;
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const int tc = wn * WTN + j * 32;  // tile column of the block
+      const bool gate = GEGLU && tc >= BN / 2;
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const int c = 8 * g + 4 * lg;
+        uint16_t o[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int gcol = n0 + tc + c + e - (gate ? BN / 2 : 0);
+          float bv = 0.f;
+          if (bias != nullptr && gcol < N) bv = to_f<BF16>(bias[gcol + (gate ? N : 0)]);
+          o[e] = from_f<BF16>(acc[i][j][4 * g + e] + bv);
+        }
+        *(uint2v*)(Cs + orow * BN + tc + c) =
+            uint2v{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+      }
     }
   }
-
-  // bias, one rounding, GeGLU on the lane's (value, gate) pair, the residual,
-  // as the other kernels; lane l holds row l % 32 and columns 8*g + 4*(l/32) +
-  // {0..3} of each column block
-  if (row >= M) return;
+  __syncthreads();
+  if constexpr (!GEGLU) {
+    if (!ypan) {
+      write_tile<BF16, BM, BN, NT>(Cs, m0, n0, M, N, R, ldr, Y, ldy);
+      return;
+    }
+  }
+  // GeGLU, or panel order (N % 16 == 0, no residual: 32 rows of a 16-byte
+  // column are 512 contiguous bytes, so the lanes go down the rows)
+  constexpr int CPR = BNO / 8;
+  for (int q = tid; q < BM * CPR; q += NT) {
+    const int r = ypan ? q % BM : q / CPR, c = (ypan ? q / BM : q % CPR) * 8, gm = m0 + r, gn = n0 + c;
+    if (gm >= M || gn >= N) continue;
+    uint4v o = *(const uint4v*)(Cs + r * BN + c);
+    if constexpr (GEGLU) {
+      const uint4v g = *(const uint4v*)(Cs + r * BN + BNO + c);
+      uint32_t res[4] = {0, 0, 0, 0};
+      if (R != nullptr) {
+        if (gn + 8 <= N) {
+          const uint4v rv = *(const uint4v*)(R + (int64_t)gm * ldr + gn);
 #pragma unroll
-  for (int j = 0; j < TNO; j++) {
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-      const int col = n0 + 32 * j + 8 * g + 4 * lg;
-      if (col >= N) continue;
-      const bool whole = col + 4 <= N;
-      const uint32_t bw[2] = {rb[j][g].x, rb[j][g].y}, bgw[2] = {rbg[j][g].x, rbg[j][g].y};
-      const uint32_t rw[2] = {rres[j][g].x, rres[j][g].y};
-      uint16_t o[4];
+          for (int e = 0; e < 4; e++) res[e] = rv[e];
+        } else {
+          for (int e = 0; gn + e < N; e++) res[e >> 1] |= (uint32_t)R[(int64_t)gm * ldr + gn + e] << (16 * (e & 1));
+        }
+      }
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        float bv = 0.f, bg = 0.f;
-        if (bias != nullptr) {
-          if (whole && bvec) {
-            bv = to_f<BF16>((bw[e >> 1] >> (16 * (e & 1))) & 0xffff);
-            if constexpr (GEGLU) bg = to_f<BF16>((bgw[e >> 1] >> (16 * (e & 1))) & 0xffff);
-          } else if (col + e < N) {
-            bv = to_f<BF16>(bias[col + e]);
-            if constexpr (GEGLU) bg = to_f<BF16>(bias[N + col + e]);
-          }
+        uint32_t h[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+          const float val = to_f<BF16>((o[e] >> (16 * k)) & 0xffff), gt = to_f<BF16>((g[e] >> (16 * k)) & 0xffff);
+          h[k] = from_f<BF16>(pin_f32(gelu_fast(val) * gt));  // the f32 product, then one rounding
+          if (R != nullptr) h[k] = from_f<BF16>(to_f<BF16>(h[k]) + to_f<BF16>((res[e] >> (16 * k)) & 0xffff));
         }
-        float v = to_f<BF16>(from_f<BF16>(acc[j][4 * g + e] + bv));
-        if constexpr (GEGLU) {
-          const float gt = to_f<BF16>(from_f<BF16>(acc[j + TN / 2][4 * g + e] + bg));
-          v = pin_f32(gelu_fast(v) * gt);  // the f32 product, then one rounding to the storage type
-        }
-        o[e] = from_f<BF16>(v);
-        if (R != nullptr) {
-          const uint16_t r16 = whole ? (uint16_t)((rw[e >> 1] >> (16 * (e & 1))) & 0xffff)
-                                     : (col + e < N ? R[(int64_t)row * ldr + col + e] : (uint16_t)0);
-          o[e] = from_f<BF16>(to_f<BF16>(o[e]) + to_f<BF16>(r16));
-        }
+        o[e] = h[0] | (h[1] << 16);
       }
-      // row-major, or panel order (ypan: N % 16 == 0, so the 4 columns are
-      // whole and 8 bytes of one 16-byte chunk of a 1 KB block)
-      uint16_t* yp = ypan ? Y + ((int64_t)(row >> 5) * (N >> 4) + (col >> 4)) * 512 +
-                                (((col >> 3) & 1) * 32 + (row & 31)) * 8 + (col & 7)
-                          : Y + (int64_t)row * ldy + col;
-      if (whole) {
-        *(uint2v*)yp = uint2v{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
-      } else {
-        for (int e = 0; col + e < N; e++) yp[e] = o[e];
-      }
+    }
+    uint16_t* yp = ypan ? Y + ((int64_t)(gm >> 5) * (N >> 4) + (gn >> 4)) * 512 + (((gn >> 3) & 1) * 32 + (gm & 31)) * 8
+                        : Y + (int64_t)gm * ldy + gn;
+    if (gn + 8 <= N) {
+      *(uint4v*)yp = o;
+    } else {
+      for (int e = 0; e < 8 && gn + e < N; e++) yp[e] = (uint16_t)(o[e >> 1] >> (16 * (e & 1)));
     }
   }
 }
@@ -1371,6 +1401,13 @@ void launch_mfma(hipStream_t st, const uint16_t* x, int64_t ldx, const uint16_t*
   kern<<<tiles_m * tiles_n, WM * WN * 64, lds, st>>>(x, ldx, w, qw, bias, r, ldr, y, ldy, M, N, K, tiles_n);
 }
 
+// Blocks per XCD of the large-M kernel, and the tiles the busiest one walks:
+// an XCD owns whole row panels, so it may hold more than an eighth of the tiles.
+inline int64_t arow_tiles_per_xcd(int64_t M, int64_t tiles_n) { return ((M + 255) / 256 + 7) / 8 * tiles_n; }
+inline int64_t arow_rounds(int64_t M, int64_t tiles_n, int cus) {
+  return (arow_tiles_per_xcd(M, tiles_n) + cus / 8 - 1) / (cus / 8);
+}
+
 template <int BN, bool BF16, bool GEGLU, bool KTAIL, bool QKV = false>
 void launch_arow(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int64_t ldx, const uint16_t* w,
                  const uint16_t* bias, const uint16_t* r, int64_t ldr, uint16_t* y, int64_t ldy, int M, int N, int K,
@@ -1384,7 +1421,10 @@ void launch_arow(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int64
   // row panels).
   const int KT = (K + 63) / 64;
   const bool stream = KT % 6 == 0 || KT >= 12;
-  int grid = stream ? (tiles < cus ? tiles : cus) / 8 * 8 : 8 * (((tiles_m + 7) / 8) * tiles_n);
+  // (streaming: never fewer blocks than the busiest XCD has tiles to run side by
+  // side: 5120 x 768 x 768, 20 row panels, 38 -> 23 us)
+  const int64_t per_xcd = arow_tiles_per_xcd(M, tiles_n);
+  const int grid = (int)(8 * (stream && per_xcd > cus / 8 ? cus / 8 : per_xcd));
   HB_REQUIRE(grid >= 8, "hb_linear: large-M GEMM needs at least 8 tiles");
   constexpr int RG = (BNO / 8 + 7) / 8;
   // W tiles and the C tile
@@ -1398,83 +1438,85 @@ void launch_arow(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int64
                                (pan & HB_Y_PANEL) ? 1 : 0, qk);
 }
 
-// Waves per slab block (each takes 32 rows of X): two for slabs of at most
-// 32 x 768 weights when those blocks fit one per CU, else four.  A launch
-// spread over more CUs finishes sooner although X and the slabs are then read
-// by more blocks (the k16 order per output is the same for any count), as
-// long as a wave's share of the slab stays small: at two waves the 64-row
-// GeGLU slab and the K = 1152 slab measured slower, and one wave per block
-// (the whole slab to fetch) slower still.
-inline int slab_waves(int64_t M, int64_t tiles_n, int64_t slab_elems, int cus) {
-  return slab_elems <= 32 * 768 && tiles_n * ((M + 63) / 64) <= cus ? 2 : 4;
+template <int BM, int BN, int WM, int WN, int NST, bool BF16, bool GEGLU>
+void launch_ring_t(hipStream_t st, unsigned pan, const uint16_t* x, int64_t ldx, const uint16_t* w, const uint16_t* bias,
+                   const uint16_t* r, int64_t ldr, uint16_t* y, int64_t ldy, int M, int N, int K) {
+  constexpr int BNO = GEGLU ? BN / 2 : BN;
+  constexpr int lds = NST * (BM + BN) * 128;
+  static_assert(lds >= BM * BN * 2 && lds <= 160 * 1024, "the C tile reuses the ring");
+  auto kern = gemm_ring<BM, BN, WM, WN, NST, BF16, GEGLU>;
+  static std::atomic<uint64_t> attr{0};
+  once_per_device(attr, [&] {
+    HB_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  });
+  const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BNO - 1) / BNO;
+  HB_REQUIRE(tiles_m * tiles_n < (1ll << 31), "hb_linear: too many tiles");
+  kern<<<(unsigned)(tiles_m * tiles_n), WM * WN * 64, lds, st>>>(x, ldx, w, bias, r, ldr, y, ldy, M, N, K, (int)tiles_n,
+                                                                  (pan & HB_X_PANEL) ? 1 : 0, (pan & HB_Y_PANEL) ? 1 : 0);
 }
 
-// Small-M launcher for 16-bit weights: slabs of 32 (GeGLU: 64) W rows, 64
-// or 128 rows of X per block (slab_waves).  P (X steps held in registers)
-// is the largest of 48, 36, 32, 24, 16 and 4 that divides K/16.
-// LDS bytes of a slab block: the f16 slab of 32 tn rows, and for quantized
-// weights the slab's codes and its scales (and zeros: aff), G per row in
-// 4-byte slots
-inline int64_t slab_lds(int64_t K, int tn, int qb, bool aff, int64_t G) {
-  const int64_t sr = 32 * tn;
-  return sr * K * 2 + (qb ? sr * K * qb / 8 + sr * G * 4 * (aff ? 2 : 1) : 0);
+// Operands the ring kernel's 32-bit offsets reach.
+inline bool ring_ok(int64_t ldx, int64_t K) { return K % 64 == 0 && K < (1 << 22) && ldx < (1 << 22); }
+
+// The ring's tile, by how many of each shape the call has (wrows: weight rows;
+// us, f16, back to back; 64 x 64 / 128 x 64 / 64 x 64 with three stages / 128 x
+// 256, and what the kernels before it took):
+// - 64 x 64, four stages, while they fit one per CU: 128 x 768 x 768 (24 tiles)
+//   5.8 / 7.4 / 6.3 / 15.0 (9.7), 256 x 2304 x 768 (144) 5.9 / 7.4 / 6.6 / 14.3
+//   (11.5); from K = 2048 five stages, as K chains of 48 stages wait for memory:
+//   512 x 768 x 3072 16.1 -> 13.7 (32.5);
+// - 128 x 64 while those fit: 512 x 3072 x 768 (192) 10.7 / 8.3 / 11.3 / 14.7
+//   (12.1), 768 x 2304 x 768 (216) 8.7 / 8.4 / 9.3 / 15.4 (12.3);
+// - 128 x 256, one round of them that fills more than half the CUs: 2048 x 2304
+//   x 768 (144) 19.4 / 21.9 / 18.7 / 17.6 (21.9), 3072 x 2304 x 768 (216) 24.9 /
+//   28.0 / 25.6 / 19.7 (23.6);
+// - else 64 x 64 with three stages, three blocks per CU: 1024 x 3072 x 768
+//   15.4 / 15.7 / 12.6 / 19.0 (16.4), 4096 x 768 x 768 12.1 / 14.0 / 11.1 / 15.7
+//   (25.6, the large-M kernel).
+template <bool BF16, bool GEGLU>
+void launch_ring(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int64_t ldx, const uint16_t* w,
+                 const uint16_t* bias, const uint16_t* r, int64_t ldr, uint16_t* y, int64_t ldy, int M, int N, int K) {
+  const int64_t wrows = GEGLU ? 2 * (int64_t)N : N;
+  auto tiles = [&](int bm, int bn) { return ((M + (int64_t)bm - 1) / bm) * ((wrows + bn - 1) / bn); };
+  const int64_t wide = tiles(128, 256);
+  if (tiles(64, 64) <= cus && K < 2048)
+    launch_ring_t<64, 64, 2, 2, 4, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
+  else if (tiles(64, 64) <= cus)
+    launch_ring_t<64, 64, 2, 2, 5, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
+  else if (tiles(128, 64) <= cus)
+    launch_ring_t<128, 64, 4, 2, 4, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
+  else if (wide > cus / 2 && wide <= cus)
+    launch_ring_t<128, 256, 4, 4, 3, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
+  else
+    launch_ring_t<64, 64, 2, 2, 3, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
 }
 
-// Quantized weights on the slab kernel: f16 scales, groups a multiple of 8
-// (a chunk of 8 weights in one group), K / 16 a multiple of 48 or 36 (the
-// register depths instantiated for them), and the block's LDS within bounds.
-inline bool qslab_ok(int64_t K, int tn, int qb, bool aff, const QW& qw) {
-  return qw.group % 8 == 0 && ((K / 16) % 48 == 0 || (K / 16) % 36 == 0) &&
-         slab_lds(K, tn, qb, aff, qw.G) <= 160 * 1024;
+// From M = 4096, the ring kernel still beats the large-M one where its 256 x 192
+// tiles are few (N = 768 at M = 4096: 64 tiles): both as measured, in us: the
+// large-M kernel a fixed 7.5 and 3 + 0.016 K a round, the ring 4 and 3.4 per
+// 64 x 64 tile and CU at K = 768.  Both sides (large-M with panel-order X /
+// ring): 4096 x 768 x 768 22.8 / 15.4, 6144 x 768 x 1152 28.5 / 26.7, 8192 x 768
+// x 768 23.5 / 23.6, 4096 x 2304 x 768 25.3 / 33.6, 6144 x 768 x 3072 55.6 / 58.2.
+inline bool ring_beats_arow(int64_t M, int64_t N_out, int64_t K, bool geglu, int bn, int cus) {
+  const int64_t wrows = geglu ? 2 * N_out : N_out, bno = geglu ? bn / 2 : bn;
+  const double per_cu = (double)(((M + 63) / 64) * ((wrows + 63) / 64)) / cus;
+  const double ring = 4 + 3.4 * (K / 768.0) * (per_cu > 1 ? per_cu : 1);
+  const double arow = 7.5 + (double)arow_rounds(M, (N_out + bno - 1) / bno, cus) * (3 + 0.016 * K) * (bn / 192.0);
+  return ring < arow;
 }
 
-template <int TN, bool BF16, bool GEGLU, int QB = 0, bool AFF = false>
-void launch_slab_t(hipStream_t st, int cus, QW qw, const uint16_t* x, int64_t ldx, const uint16_t* w,
-                   const uint16_t* bias, const uint16_t* r, int64_t ldr, uint16_t* y, int64_t ldy, int M, int N,
-                   int K, unsigned pan) {
-  constexpr int TNO = GEGLU ? TN / 2 : TN;
-  const int tiles_n = (N + 32 * TNO - 1) / (32 * TNO);
-  const int nw = slab_waves(M, tiles_n, (int64_t)32 * TN * K, cus), chunks = (M + 32 * nw - 1) / (32 * nw);
-  const int64_t lds = slab_lds(K, TN, QB, AFF, QB ? qw.G : 0);
-  HB_REQUIRE(lds <= 160 * 1024, "hb_linear: weight slab too large for LDS");
-  const int S = K / 16;
-  auto go = [&](auto kern) {
-    static std::atomic<uint64_t> attr{0};
-    once_per_device(attr, [&] {
-      HB_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    });
-    kern<<<tiles_n * chunks, 64 * nw, (size_t)lds, st>>>(x, ldx, w, qw, bias, r, ldr, y, ldy, M, N, K, chunks,
-                                                          (pan & HB_X_PANEL) ? 1 : 0, (pan & HB_Y_PANEL) ? 1 : 0);
-  };
-  if constexpr (QB != 0) {
-    HB_REQUIRE(S % 48 == 0 || S % 36 == 0, "hb_linear: quantized slab needs K a multiple of 768 or 576");
-    if (S % 48 == 0) go(gemm_slab<TN, 48, BF16, GEGLU, QB, AFF>);
-    else go(gemm_slab<TN, 36, BF16, GEGLU, QB, AFF>);
-  } else {
-    if (S % 48 == 0) go(gemm_slab<TN, 48, BF16, GEGLU>);
-    else if (S % 36 == 0) go(gemm_slab<TN, 36, BF16, GEGLU>);
-    else if (S % 32 == 0) go(gemm_slab<TN, 32, BF16, GEGLU>);
-    else if (S % 24 == 0) go(gemm_slab<TN, 24, BF16, GEGLU>);
-    else if (S % 16 == 0) go(gemm_slab<TN, 16, BF16, GEGLU>);
-    else go(gemm_slab<TN, 4, BF16, GEGLU>);
-  }
-}
-
-// The slab kernel pays off while its blocks fit one per CU: its X fragment
-// loads (32 rows x 32 bytes each) are bound by the CU's L1 (about 15 bytes
-// per clock for that pattern), so two blocks on one CU take twice as long and
-// the 128 x 128 kernel, which stages X through LDS, is faster from there on.
-inline bool slab_path(int64_t M, int64_t N_out, int64_t K, bool geglu, int cus) {
+// Calls below M = 4096 that take panel-order operands (laya_hip.h): 16-bit
+// weights, and few enough rows that the producer's panel costs nothing.
+inline bool small_panel_path(int64_t M, int64_t N_out, int64_t K, bool geglu, int cus) {
   const int64_t tiles_n = (N_out + 31) / 32, chunks = (M + 127) / 128;
   return K % 64 == 0 && K * 32 * (geglu ? 2 : 1) * 2 <= 160 * 1024 && tiles_n * chunks <= cus;
 }
 
-// The large-M kernel runs for M >= 4096.  It and the small-M slab kernel
-// (16-bit weights) take panel-order operands; the entry points check that
-// the call takes one of them before dispatching.
+// Calls of the large-M kernel's size (the ring kernel takes those it beats it
+// at); both take panel-order operands.
 inline bool arow_path(int64_t M) { return M >= 4096; }
 
-// Below M = 4096, without the slab kernel: 128 x 64 tiles (instead of
+// Below M = 4096 with K % 64 != 0: 128 x 64 tiles (instead of
 // 128 x 128) where 128 x 128 tiles would leave the GPU short of blocks.
 // N_out: output columns (GeGLU: value / gate pairs).
 inline bool thin_tiles(int64_t M, int64_t N_out, bool geglu, int cus) {
@@ -1486,16 +1528,21 @@ template <bool BF16, bool GEGLU, int QB, bool AFF, bool SF32>
 void mfma_dispatch(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int64_t ldx, const uint16_t* w,
                           QW qw, const uint16_t* bias, const uint16_t* r, int64_t ldr, uint16_t* y, int64_t ldy, int M,
                           int N, int K) {
-  // large M: persistent 256 x 192 tiles with register-resident A rows (16-bit
-  // weights: hb_qlinear dequantizes a quantized weight once and calls the
-  // 16-bit path at large M); small M: weight-stationary slabs, else 128 x 128
-  // tiles.  K % 64 != 0 takes the large-M variant with a K tail.
+  // K % 64 == 0: the ring kernel, or from M = 4096 persistent 256 x 192 tiles with
+  // register-resident A rows (hb_qlinear dequantizes a quantized weight once and
+  // calls the 16-bit path).  Other K: the large-M variant with a K tail, below M
+  // = 4096 the 128-row tiles.
   if constexpr (QB == 0) {
+    // 128-column tiles of the large-M kernel where N is a multiple of 128 and
+    // not of 192 (N = 1024: 8 whole tiles instead of 5 1/3 of 192 columns)
+    const bool n128 = !GEGLU && N % 192 != 0 && N % 128 == 0;
+    if (ring_ok((pan & HB_X_PANEL) ? K : ldx, K) && (!arow_path(M) || ring_beats_arow(M, N, K, GEGLU, n128 ? 128 : 192, cus))) {
+      launch_ring<BF16, GEGLU>(st, cus, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
+      return;
+    }
     if (arow_path(M)) {
-      // 128-column tiles where N is a multiple of 128 and not of 192 (N =
-      // 1024: 8 whole tiles instead of 5 1/3 of 192 columns)
       if constexpr (!GEGLU) {
-        if (N % 192 != 0 && N % 128 == 0) {
+        if (n128) {
           if (K % 64 == 0)
             launch_arow<128, BF16, false, false>(st, cus, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
           else
@@ -1513,25 +1560,11 @@ void mfma_dispatch(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int
     HB_REQUIRE(!arow_path(M), "hb_qlinear: large-M quantized weights are dequantized before the GEMM");
   }
   {
-    if constexpr (QB == 0 || !SF32) {
-      if (slab_path(M, N, K, GEGLU, cus) && (QB == 0 || qslab_ok(K, GEGLU ? 2 : 1, QB, AFF, qw))) {
-        launch_slab_t<GEGLU ? 2 : 1, BF16, GEGLU, QB, AFF>(st, cus, qw, x, ldx, w, bias, r, ldr, y, ldy, M, N, K,
-                                                          pan);
-        return;
-      }
-    }
     HB_REQUIRE(pan == 0, "hb_linear: panel-order operands on a kernel that does not take them");
-    // Tiles of 128 x 64 (waves of 32 x 64) where 128 x 128 tiles would
-    // leave the GPU short of blocks: the K stages of a block run one after
-    // another (each one's loads, LDS staging and barrier), so a launch with
-    // few blocks is bound by that chain; halving the tile halves the work
-    // of each stage.  Measured (16-bit, M = 2048): attn Wo 18.2 -> 14.3 us,
-    // mlp Wo 22.9 -> 18.1 us; at M = 3072 the 2304-column shapes are faster
-    // with 128 x 128 tiles (27.0 against 32.8 us).  Every output keeps its
-    // MFMA sequence and epilogue, so the bits do not change.  Quantized
-    // weights take the same rule (their loader dequantizes each stage of
-    // the thinner W tile; hb_qlinear calls with a quantized weight wherever
-    // these tiles are taken below M = 4096).
+    // Tiles of 128 x 64 (waves of 32 x 64) where 128 x 128 tiles would leave the
+    // GPU short of blocks: the K stages of a block run one after another, so a
+    // launch with few blocks is bound by that chain.  Every output keeps its
+    // MFMA sequence and epilogue, so the bits do not change.
     if (thin_tiles(M, N, GEGLU, cus)) {
       launch_mfma<128, 64, 4, 1, BF16, GEGLU, QB, AFF, SF32>(st, x, ldx, w, qw, bias, r, ldr, y, ldy, M, N, K);
       return;

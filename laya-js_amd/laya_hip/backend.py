@@ -20,7 +20,7 @@ Design (MI355X-first, not a port of any reference backend):
   [B, L, H*D] (modernbert/src/index.ts:352) is free.
 - `layerNorm` and `geglu` of a pending linear are pending too.  When their
   first consumer is a linear layer that reads panel order (16-bit, K % 64 ==
-  0, and M >= 4096 or, with 16-bit weights, the small-M slab kernel) they
+  0, and M >= 4096 or, with 16-bit weights, few rows) they
   are written in panel order (laya_hip.h: 32 x 16 blocks in MFMA
   operand order), which the GEMM loads a whole block per instruction; any
   other reader gets a row-major copy (hb_panel_unpack).  Same values, bit
@@ -146,14 +146,14 @@ class HipTensor:
 
 # ------------------------------------------------------------------ pending work
 
-PANEL_MIN_M = 4096  # the large-M GEMM; below it the small-M slab kernel also takes panel-order operands
-SLAB_LDS = 160 * 1024  # the slab kernel's LDS: 64 * K bytes per 32 output columns (x2 with GeGLU)
+PANEL_MIN_M = 4096  # from here on, and for small calls (_small_panel_path), linears take panel-order operands
+PANEL_W_BYTES = 160 * 1024  # their bound on 32 output columns of weights: 64 * K bytes (x2 with GeGLU)
 
 
-def _slab_path(M: int, n_out: int, K: int, geglu: bool, cus: int) -> bool:
-    """hb_linear takes the small-M slab kernel (16-bit weights, M < 4096):
-    the conditions of slab_path in csrc/gemm_kernels.h."""
-    return (M < PANEL_MIN_M and K % 64 == 0 and 64 * K * (2 if geglu else 1) <= SLAB_LDS
+def _small_panel_path(M: int, n_out: int, K: int, geglu: bool, cus: int) -> bool:
+    """hb_linear takes panel-order operands below M = 4096 (16-bit weights):
+    the conditions of small_panel_path in csrc/gemm_kernels.h."""
+    return (M < PANEL_MIN_M and K % 64 == 0 and 64 * K * (2 if geglu else 1) <= PANEL_W_BYTES
             and -(-n_out // 32) * -(-M // 128) <= cus)
 
 
@@ -257,13 +257,13 @@ class _PendingLinear:
 
     def takes_panel(self, epi: int) -> bool:
         """The launch with epilogue `epi` takes a kernel that reads and
-        writes panel order: the large-M one, or (16-bit weights) the slab."""
+        writes panel order: M >= 4096, or (16-bit weights) a small call."""
         if self.arow_ok:
             return True
         M, K = self.x[1], self.x[2]
         geglu = bool(epi & F.HB_EPI_GEGLU)
         n_out = self.N // 2 if geglu else self.N
-        return self.operands_ok and self.q is None and _slab_path(M, n_out, K, geglu, self.be.cus)
+        return self.operands_ok and self.q is None and _small_panel_path(M, n_out, K, geglu, self.be.cus)
 
     def fork(self, epi: int) -> "_PendingLinear":
         """The same product with epilogue `epi` (own references)."""
@@ -1504,15 +1504,15 @@ class HipBackend:
 
     def _panel_for(self, x: HipTensor, w: Optional[HipTensor] = None, q=None) -> Optional[_PanelRows]:
         """The panel-order form of x when this linear layer takes a kernel
-        that reads it: the large-M one, or for 16-bit weights the small-M slab
-        kernel as the launch without an epilogue takes it (weights side
+        that reads it: M >= 4096, or for 16-bit weights a small call, as the
+        launch without an epilogue takes it (weights side
         checked here, x side by _as_panel; a launch that ends up taking
         another kernel unpacks x)."""
         if x.dtype not in ("f16", "bf16") or not x.shape:
             return None
         M = _numel(x.shape[:-1])
         if M < PANEL_MIN_M and (q is not None or w is None
-                                or not _slab_path(M, w.shape[0], x.shape[-1], False, self.cus)):
+                                or not _small_panel_path(M, w.shape[0], x.shape[-1], False, self.cus)):
             return None
         if x._lazy is None or isinstance(x._lazy, _PendingRope):
             return None
