@@ -1461,7 +1461,10 @@ inline bool ring_ok(int64_t ldx, int64_t K) { return K % 64 == 0 && K < (1 << 22
 // The ring's tile, by how many of each shape the call has (wrows: weight rows;
 // us, f16, back to back; 64 x 64 / 128 x 64 / 64 x 64 with three stages / 128 x
 // 256, and what the kernels before it took):
-// - 64 x 64, four stages, while they fit one per CU: 128 x 768 x 768 (24 tiles)
+// - 32 x 64, six stages, while they fit one per CU: with weights that come from
+//   HBM (a model's layers in turn), where the bytes a launch has in flight count,
+//   128 x 2304 x 768 7.9 -> 6.7, 128 x 2304 x 768 GeGLU 8.2 -> 7.0 against 64 x 64;
+// - 64 x 64, four stages, while those fit: 128 x 768 x 768 (24 tiles)
 //   5.8 / 7.4 / 6.3 / 15.0 (9.7), 256 x 2304 x 768 (144) 5.9 / 7.4 / 6.6 / 14.3
 //   (11.5); from K = 2048 five stages, as K chains of 48 stages wait for memory:
 //   512 x 768 x 3072 16.1 -> 13.7 (32.5);
@@ -1479,7 +1482,9 @@ void launch_ring(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int64
   const int64_t wrows = GEGLU ? 2 * (int64_t)N : N;
   auto tiles = [&](int bm, int bn) { return ((M + (int64_t)bm - 1) / bm) * ((wrows + bn - 1) / bn); };
   const int64_t wide = tiles(128, 256);
-  if (tiles(64, 64) <= cus && K < 2048)
+  if (tiles(32, 64) <= cus)
+    launch_ring_t<32, 64, 1, 2, 6, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
+  else if (tiles(64, 64) <= cus && K < 2048)
     launch_ring_t<64, 64, 2, 2, 4, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
   else if (tiles(64, 64) <= cus)
     launch_ring_t<64, 64, 2, 2, 5, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);

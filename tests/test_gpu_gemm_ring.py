@@ -13,11 +13,11 @@ from oracle import cpu_ref as cr
 pytestmark = pytest.mark.gpu
 TOL = {"f16": 2e-3, "bf16": 8e-3}
 
-# (M, N, K): one 64 x 64 tile and less; a few with row and column remainders;
-# K long enough for five stages; K shorter than the ring; 128 x 64 tiles;
-# 64 x 64 with three stages; 128 x 256
-SHAPES = [(1, 8, 64), (65, 72, 128), (130, 200, 768), (70, 136, 2112), (900, 1304, 192), (1030, 3000, 64),
-          (2100, 2120, 128), (4100, 768, 256)]
+# (M, N, K): one 32 x 64 tile and less; a few with row and column remainders;
+# K shorter than the ring and long; 64 x 64 with four stages and, from K = 2048,
+# five; 128 x 64 tiles; 64 x 64 with three stages; 128 x 256
+SHAPES = [(1, 8, 64), (65, 72, 128), (130, 200, 768), (70, 136, 2112), (520, 1032, 192), (520, 1032, 2112),
+          (900, 1304, 192), (1030, 3000, 64), (2100, 2120, 128), (4100, 768, 256)]
 
 
 @pytest.fixture(scope="module")
@@ -54,7 +54,7 @@ def test_ring_tiles(b, M, N, K, dtype):
         np.testing.assert_array_equal(read32(b, b.linear(xi, W, B))[0], got[i])
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (65, 40, 128), (300, 648, 2112), (900, 648, 192), (1030, 1504, 64),
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (65, 40, 128), (300, 648, 2112), (520, 520, 192), (900, 648, 192), (1030, 1504, 64),
                                    (2100, 1064, 128)])
 def test_ring_geglu(b, M, N, K):
     """Value and gate columns in one tile, in waves of their own: the bits of
