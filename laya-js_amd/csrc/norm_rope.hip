@@ -160,7 +160,8 @@ __global__ __launch_bounds__(kLnNT) void layernorm_panel_kernel(const uint16_t* 
 
 // f32 rows of 256 * G values: one row per wave, held in registers (16-byte
 // loads), so it is read once.  Memory-bound; the generic kernel below reads
-// the row three times, 4 bytes a lane, and each pass waits for the last.
+// the row three times, 4 bytes a lane, and each pass waits for the last
+// (4096 x 768 18.5 -> 6.5 us, 3.9 TB/s; 93 x 768 15.3 -> 4.6 us).
 template <int G, int PK>
 __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restrict__ x, int64_t ldx,
                                                             const void* __restrict__ w, const void* __restrict__ b,
