@@ -1433,14 +1433,14 @@ static void sdpa_impl(uintptr_t ctx, int dt, uintptr_t q, const int64_t* qs, uin
   if (fast) {
     int nqt = (int)((Lq + kBQ - 1) / kBQ);
     uint8_t* info = (uint8_t*)mask_info;
-    uint8_t* tmp = nullptr;
+    CallScratch tmp(ctx);
     if (mask) {
       if (!info) {
         HB_REQUIRE(!noalloc, "hb_sdpa_noalloc: no mask summary");
-        tmp = (uint8_t*)pool_alloc(ctx, mask_info_bytes(B, Lq, Lk));
-        launch_mask_info(st, (const uint8_t*)mask, Ms, B, Lq, Lk, tmp);
+        HB_REQUIRE(tmp.take(mask_info_bytes(B, Lq, Lk)), "hb_sdpa: out of device memory for the mask summary");
+        info = (uint8_t*)tmp.p;
+        launch_mask_info(st, (const uint8_t*)mask, Ms, B, Lq, Lk, info);
         check_launch("hb_sdpa(mask info)");
-        info = tmp;
       }
     } else {
       info = nullptr;
@@ -1465,16 +1465,10 @@ static void sdpa_impl(uintptr_t ctx, int dt, uintptr_t q, const int64_t* qs, uin
       // From 1024 keys that every query tile reads, K is rotated once in a pass
       // of its own instead of by every block that stages it (T 2048 B 16 465 ->
       // 434, T 8192 B 1 367 -> 322 us, the pass included; T 512 B 32 50 -> 54).
-      struct PoolBlock {  // back to the pool when the call ends, by return or throw
-        uintptr_t ctx;
-        void* p;
-        ~PoolBlock() {
-          if (p) pool_free(ctx, p);  // stream-ordered: reused only by work enqueued later
-        }
-      } rotated{ctx, nullptr};
+      // (Without memory for the rotated copy the blocks rotate what they stage.)
+      CallScratch rotated(ctx);
       const int64_t kblk = (Lk + 63) / 64 * B * H;
-      if (tk && all_keys && Lk >= 1024 && kblk < ((int64_t)1 << 31)) {
-        rotated.p = pool_alloc(ctx, (size_t)(B * H * Lk * 64 * 2));
+      if (tk && all_keys && Lk >= 1024 && kblk < ((int64_t)1 << 31) && rotated.take((size_t)(B * H * Lk * 64 * 2))) {
         auto kern = dt == HB_F16 ? rope_k_kernel<false> : rope_k_kernel<true>;
         kern<<<(unsigned)kblk, 256, 0, st>>>((const uint16_t*)k, Ks, (uint16_t*)rotated.p, (int)Lk, (int)H, (int)(B * H),
                                              tk);
@@ -1498,7 +1492,6 @@ static void sdpa_impl(uintptr_t ctx, int dt, uintptr_t q, const int64_t* qs, uin
                                            sl2, tq, tk, pK, nqt, (int)H);
     }
     check_launch("hb_sdpa");
-    if (tmp) pool_free(ctx, tmp);
   } else if (sdpa_takes_f32(dt, q, qs, k, ks, v, vs, o, os, Lk, D)) {
     const int nqt = (int)((Lq + kFQ - 1) / kFQ);
     const int64_t nblk = (int64_t)nqt * H * B;

@@ -50,6 +50,22 @@ void sdpa_scratch_init(int device);
 void* pool_alloc(uintptr_t ctx, size_t bytes);
 void pool_free(uintptr_t ctx, void* p);
 
+// Pool memory that only the kernels of one call use, given back when the call
+// ends, by return or throw (stream-ordered: reused only by work enqueued
+// later).  While a graph is recorded the recorded calls share such blocks
+// among themselves, so a graph holds its largest ones once and not one per
+// call.  p is null where the device has no memory left: the caller then takes
+// a path without scratch, or fails.
+struct CallScratch {
+  uintptr_t ctx;
+  void* p = nullptr;
+  explicit CallScratch(uintptr_t c) : ctx(c) {}
+  CallScratch(const CallScratch&) = delete;
+  CallScratch& operator=(const CallScratch&) = delete;
+  ~CallScratch();
+  bool take(size_t bytes);  // once; false: no memory
+};
+
 // ------------------------------------------------------------------ dtypes
 
 typedef _Float16 f16;

@@ -401,18 +401,20 @@ extern "C" int hb_qlinear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintp
     uint16_t* Yp = (uint16_t*)y;
     int m = (int)M, n = (int)N, k = (int)K;
     const int cus0 = cu_count(ctx);
-    if (arow_path(M) || ring_ok(ldx, K) || (M >= 1024 && !thin_tiles(M, N, geglu, cus0))) {
+    const int64_t rows = geglu ? 2 * N : N;
+    CallScratch held(ctx);
+    bool dequant = arow_path(M) || ring_ok(ldx, K) || (M >= 1024 && !thin_tiles(M, N, geglu, cus0));
+    if (dequant && !held.take((size_t)(rows * K * 2))) {
+      // no memory for the copy: gemm_mfma's loader dequantizes without one
+      HB_REQUIRE(!arow_path(M), "hb_qlinear: out of device memory for the dequantized weight");
+      dequant = false;
+    }
+    if (dequant) {
       // The weight is dequantized once into a pooled 16-bit copy and the 16-bit
       // GEMM runs on it: one bandwidth-bound pass over the weight (4-6 us)
       // instead of the same work in every row tile's loader (M = 512, q4, the
       // pass included: 1152 x 768 GeGLU 20.7 -> 12.5, 768 x 1152 18.8 -> 11 us).
       // gemm_mfma dequantizes in its loader where it has few blocks.
-      const int64_t rows = geglu ? 2 * N : N;
-      struct PoolBlock {  // back to the pool when the call ends, by return or throw
-        uintptr_t ctx;
-        void* p;
-        ~PoolBlock() { pool_free(ctx, p); }  // stream-ordered: reused only by work enqueued later
-      } held{ctx, pool_alloc(ctx, (size_t)(rows * K * 2))};
       uint16_t* wd = (uint16_t*)held.p;
       const int cus = cu_count(ctx);
       if (bits == 8 && mode == 0) launch_dequant_rows<8, false>(st, cus, dt, q, wd, rows, k);

@@ -49,6 +49,7 @@ struct Context {
   // (a replay still writes them) until their graph is destroyed
   bool capturing = false;
   std::vector<void*> held;
+  std::vector<void*> call_scratch;  // live blocks that earlier calls of the recording used and later ones may
   std::map<void*, std::vector<void*>> graph_held;  // hipGraphExec_t -> held blocks
 };
 
@@ -84,6 +85,10 @@ static void require_current(const Context* c) {
                              ") on this thread first)");
 }
 
+struct OutOfMemory : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+
 void* pool_alloc(uintptr_t ctx, size_t bytes) {
   Context* c = C(ctx);
   size_t sc = size_class(bytes);
@@ -97,8 +102,8 @@ void* pool_alloc(uintptr_t ctx, size_t bytes) {
     require_current(c);
     hipError_t e = hipMalloc(&p, sc);
     if (e != hipSuccess && c->capturing)  // the retry below would synchronize the recording stream
-      throw std::runtime_error("hb_alloc: out of device memory for " + std::to_string(bytes) +
-                               " bytes while recording a graph");
+      throw OutOfMemory("hb_alloc: out of device memory for " + std::to_string(bytes) +
+                        " bytes while recording a graph");
     if (e != hipSuccess) {
       // release the cache once and retry before failing
       HB_CHECK_HIP(hipStreamSynchronize(c->stream));
@@ -109,13 +114,38 @@ void* pool_alloc(uintptr_t ctx, size_t bytes) {
       (void)hipGetLastError();
       e = hipMalloc(&p, sc);
       if (e != hipSuccess)
-        throw std::runtime_error("hb_alloc: out of device memory for " + std::to_string(bytes) + " bytes: " +
-                                 hipGetErrorString(e));
+        throw OutOfMemory("hb_alloc: out of device memory for " + std::to_string(bytes) + " bytes: " +
+                          hipGetErrorString(e));
     }
   }
   c->live[p] = sc;
   c->live_bytes += sc;
   return p;
+}
+
+bool CallScratch::take(size_t bytes) {
+  Context* c = C(ctx);
+  const size_t sc = size_class(bytes);
+  for (size_t i = 0; i < c->call_scratch.size(); i++)
+    if (c->live[c->call_scratch[i]] == sc) {  // the recording's kernels run in the order they were recorded
+      p = c->call_scratch[i];
+      c->call_scratch.erase(c->call_scratch.begin() + i);
+      return true;
+    }
+  try {
+    p = pool_alloc(ctx, bytes);
+  } catch (const OutOfMemory&) {
+    (void)hipGetLastError();  // not the launches' that follow
+    return false;
+  }
+  return true;
+}
+
+CallScratch::~CallScratch() {
+  if (!p) return;
+  Context* c = C(ctx);
+  if (c->capturing) c->call_scratch.push_back(p);
+  else pool_free(ctx, p);
 }
 
 void pool_free(uintptr_t ctx, void* p) {
@@ -403,6 +433,8 @@ int hb_capture_end(uintptr_t ctx, uintptr_t* exec) {
   c->capturing = false;
   std::vector<void*> held;
   held.swap(c->held);
+  held.insert(held.end(), c->call_scratch.begin(), c->call_scratch.end());
+  c->call_scratch.clear();
   hipGraph_t g = nullptr;
   hipError_t e = hipStreamEndCapture(c->stream, &g);
   hipGraphExec_t x = nullptr;

@@ -154,6 +154,51 @@ def test_recorded_quantized_linear_replays(b):
     b.dispose(X)
 
 
+def test_recorded_quantized_linears_share_their_weight_copies(b):
+    """Small-M quantized linears dequantize into scratch; a graph of many of
+    them holds one copy per size, not one per call, and replays as eager."""
+    from laya_hip import compose as C
+    from laya_hip.host import HostQuantized, pack_quantized
+    from oracle import cpu_ref as cr
+    rng = np.random.default_rng(10)
+    K, M, calls = 768, 96, 6
+    w = (rng.standard_normal((K, K)) * 0.02).astype(np.float32)
+    q, s, z = cr.quantize_matrix(w, K, K, 4, 64, refine=False)
+    h = HostQuantized((K, K), 4, 64, "affine", pack_quantized(q, 4), HostTensor("f16", s.shape, s.view(np.float16)),
+                      HostTensor("f16", z.shape, z.view(np.float16)))
+    Qs = [C.upload_quantized(b, h, "f16") for _ in range(2)]
+    X = b.fromHost(HostTensor("f16", (M, K), rng.standard_normal((M, K)).astype(np.float16)))
+
+    def chain():
+        x = X
+        for i in range(calls):
+            y = C.quantized_linear(b, x, Qs[i % 2])
+            if x is not X:
+                b.dispose(x)
+            x = y
+        return x
+
+    y = chain()
+    want = _bits(b, y)
+    b.dispose(y)
+    live0 = b.pool_stats()["live_bytes"]
+    g = b.capture(chain)
+    # the activations, and one 16-bit copy of the weight (size classes round up by at most 1/8)
+    assert b.pool_stats()["live_bytes"] - live0 <= (calls * M * K * 2 + K * K * 2) * 9 // 8
+    for _ in range(3):
+        np.testing.assert_array_equal(_bits(b, g.run()), want)
+        y = chain()
+        np.testing.assert_array_equal(_bits(b, y), want)
+        b.dispose(y)
+    out = g.out
+    g.destroy()
+    b.dispose(out)
+    assert b.pool_stats()["live_bytes"] == live0
+    for Q in Qs:
+        C.dispose_quantized(b, Q)
+    b.dispose(X)
+
+
 def test_recording_refuses_synchronizing_calls(b):
     """A read inside a recording is refused with a clear error (the host-side
     check runs before the stream is touched); the recording is dropped and
