@@ -602,7 +602,7 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void s
 // flight only makes those stronger); the caller waits for it (vmcnt(0)).
 __device__ __forceinline__ void buffer_to_lds16(const uint4v& rs, uint32_t voff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
-               : "memory");
+               : "memory", "m0");
 }
 typedef short short4t __attribute__((ext_vector_type(4)));
 // Transposing LDS read: within 16 lanes, lanes 4r .. 4r + 3 point at 4 x 4
