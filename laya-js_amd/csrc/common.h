@@ -53,7 +53,7 @@ void pool_free(uintptr_t ctx, void* p);
 // Pool memory that only the kernels of one call use, given back when the call
 // ends, by return or throw (stream-ordered: reused only by work enqueued
 // later).  While a graph is recorded the recorded calls share such blocks
-// among themselves, so a graph holds its largest ones once and not one per
+// among themselves, two of a size in turn, so a graph does not hold one per
 // call.  p is null where the device has no memory left: the caller then takes
 // a path without scratch, or fails.
 struct CallScratch {
