@@ -20,9 +20,8 @@
 // Backend.rope.  The output is written row-major or, for the attention output
 // projection, in the panel order of the GEMM's X operand.
 //
-// sdpa32_ring: the same for longer sequences and masks that every query
-// shares, 32 queries per wave on v_mfma_f32_32x32x16 (sdpa_impl says where the
-// line lies).  V goes to LDS by direct loads and is transposed by the LDS read;
+// sdpa32_ring: the same for more than 1024 keys, 32 queries per wave on
+// v_mfma_f32_32x32x16.  V goes to LDS by direct loads and is transposed by the LDS read;
 // K likewise, or through registers where RoPE rotates it on the way.
 //
 // sdpa_f32_mfma: the f32 path for head dim 64, on v_mfma_f32_32x32x2_f32.
@@ -1448,27 +1447,26 @@ static void sdpa_impl(uintptr_t ctx, int dt, uintptr_t q, const int64_t* qs, uin
     const float sl2 = scale * 1.4426950408889634f;
     const int64_t nblk = (int64_t)nqt * H * B;
     HB_REQUIRE(nblk < ((int64_t)1 << 31), "hb_sdpa: too many (batch, head, query tile) blocks");
-    // Which kernel: by the shape and the kind of mask only, never by the number
-    // of sequences, so that a sequence's bits do not depend on its batch.  The
-    // 32-query kernel wins where every query reads every key, or the
-    // sequence is long (its blocks are fewer and do more per tile); with a
-    // windowed mask on up to 1024 keys the 16-query one has the shorter chain
-    // per block.  us, 16 / 32 queries a wave, 12 heads (16 from T = 1024),
-    // padded below T = 1024, RoPE on both operands:
+    // Which kernel: by the number of keys only, so that a sequence's bits depend
+    // neither on its batch nor on how its mask is given (none, one row for every
+    // query, or a row per query: the two kernels sum in different orders).  Up to
+    // 1024 keys the 16-query kernel has the shorter chain per block, and with a
+    // windowed mask it is the faster one: us, 16 / 32 queries a wave, 12 heads
+    // (16 from T = 1024), padded below T = 1024, RoPE on both operands:
     //   every key:  T 128 B 1 9.0 / 9.6, T 384 B 8 18.9 / 19.3, T 512 B 4 19.0 /
     //               18.3, T 512 B 32 55.4 / 50.2, T 2048 B 16 566 / 465
     //   windowed:   T 512 B 8 23.4 / 26.3, T 512 B 32 53.0 / 53.2, T 1024 B 8
     //               59.1 / 61.3, T 2048 B 16 125 / 121
     const bool all_keys = !mask || ms[2] == 0;
-    const bool wide = Lk > 1024 || (all_keys && Lk > 384);
+    const bool wide = Lk > 1024;
     if (wide) {
-      // From 1024 keys that every query tile reads, K is rotated once in a pass
+      // Where every query tile reads every key, K is rotated once in a pass
       // of its own instead of by every block that stages it (T 2048 B 16 465 ->
       // 434, T 8192 B 1 367 -> 322 us, the pass included; T 512 B 32 50 -> 54).
       // (Without memory for the rotated copy the blocks rotate what they stage.)
       CallScratch rotated(ctx);
       const int64_t kblk = (Lk + 63) / 64 * B * H;
-      if (tk && all_keys && Lk >= 1024 && kblk < ((int64_t)1 << 31) && rotated.take((size_t)(B * H * Lk * 64 * 2))) {
+      if (tk && all_keys && kblk < ((int64_t)1 << 31) && rotated.take((size_t)(B * H * Lk * 64 * 2))) {
         auto kern = dt == HB_F16 ? rope_k_kernel<false> : rope_k_kernel<true>;
         kern<<<(unsigned)kblk, 256, 0, st>>>((const uint16_t*)k, Ks, (uint16_t*)rotated.p, (int)Lk, (int)H, (int)(B * H),
                                              tk);

@@ -1,5 +1,5 @@
-"""16-bit attention on 32-query waves (more than 1024 keys, or more than 384
-that every query sees): tile remainders, masks whose rows are and are not
+"""16-bit attention on either side of 1024 keys (16-query waves up to there,
+32-query waves from there): tile remainders, masks whose rows are and are not
 16-byte aligned, RoPE on the way to LDS and in a pass of its own, row-major and
 panel-order output, through the contract and the C ABI.
 
@@ -43,7 +43,8 @@ def _mask(rng, B, L, kind):
 
 
 CASES = [(385, None, 0), (448, "full", 1), (449, "full", 1), (577, "full", 0), (1023, "full", 1), (1024, "full", 1),
-         (1025, "sliding", 1), (1040, "sliding", 1), (1027, "sliding", 0), (1090, None, 1)]
+         (1025, "sliding", 1), (1040, "sliding", 1), (1027, "sliding", 0), (1090, None, 1), (1025, "full", 0),
+         (1088, "full", 1), (1217, "full", 1), (1663, None, 0)]
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
@@ -77,6 +78,25 @@ def test_sdpa_long(b, L, kind, rope, dtype):
         q1, k1 = b.rope(q1, 10000.0), b.rope(k1, 10000.0)
     M1 = None if mask is None else b.fromHost(HostTensor("bool", (1,) + mask.shape[1:], mask.data.reshape(mask.shape)[1:]))
     np.testing.assert_array_equal(got[1:], read32(b, b.sdpa(q1, k1, v1, M1, 0.125)))
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("L", [128, 385, 512, 1024, 1025, 1100])
+def test_bits_do_not_depend_on_the_form_of_the_mask(b, L, dtype):
+    """A padding mask as one row per sequence and spelt out per query, and an
+    all-true mask and none, give the same bits: the kernel is chosen by the
+    number of keys alone."""
+    B, H = 2, 3
+    rng = np.random.default_rng(L)
+    q, k, v = _views(b, rng.standard_normal((B, L, 3, H, 64)).astype(np.float32), dtype)
+    key = np.ones((B, 1, 1, L), np.uint8)
+    key[1, ..., L - L // 3:] = 0
+
+    def run(m):
+        M = None if m is None else b.fromHost(HostTensor("bool", m.shape, np.ascontiguousarray(m)))
+        return read32(b, b.sdpa(b.rope(q, 10000.0), b.rope(k, 10000.0), v, M, 0.125))
+    np.testing.assert_array_equal(run(key), run(np.broadcast_to(key, (B, 1, L, L))))
+    np.testing.assert_array_equal(run(None), run(np.ones((B, 1, 1, L), np.uint8)))
 
 
 @pytest.mark.parametrize("L", [449, 1056])
