@@ -1460,13 +1460,19 @@ static void sdpa_impl(uintptr_t ctx, int dt, uintptr_t q, const int64_t* qs, uin
     const bool all_keys = !mask || ms[2] == 0;
     const bool wide = Lk > 1024;
     if (wide) {
-      // Where every query tile reads every key, K is rotated once in a pass
-      // of its own instead of by every block that stages it (T 2048 B 16 465 ->
-      // 434, T 8192 B 1 367 -> 322 us, the pass included; T 512 B 32 50 -> 54).
+      // Where every query tile reads every key, K is rotated once in a pass of
+      // its own instead of by every block that stages it (T 2048 B 16 465 -> 434,
+      // T 8192 B 1 367 -> 322 us, the pass included), if that is shared by eight
+      // query tiles, or the pass is small against the chain of tiles whose
+      // rotations it takes out.  us, in the blocks / in a pass, 12 heads:
+      //   queries x keys  1024 x 2048 B 16 183 / 163, 512 x 2048 B 16 padded 75 /
+      //   78, 128 x 4096 B 16 98 / 141, 1 x 2048 B 64 90 / 191; few (b, h):
+      //   1 x 2048 B 1 41 / 38, 256 x 4096 B 4 95 / 80, 1 x 8192 B 4 176 / 146
       // (Without memory for the rotated copy the blocks rotate what they stage.)
       CallScratch rotated(ctx);
       const int64_t kblk = (Lk + 63) / 64 * B * H;
-      if (tk && all_keys && kblk < ((int64_t)1 << 31) && rotated.take((size_t)(B * H * Lk * 64 * 2))) {
+      const bool pass = tk && all_keys && (nqt >= 8 || B * H <= 64);
+      if (pass && kblk < ((int64_t)1 << 31) && rotated.take((size_t)(B * H * Lk * 64 * 2))) {
         auto kern = dt == HB_F16 ? rope_k_kernel<false> : rope_k_kernel<true>;
         kern<<<(unsigned)kblk, 256, 0, st>>>((const uint16_t*)k, Ks, (uint16_t*)rotated.p, (int)Lk, (int)H, (int)(B * H),
                                              tk);

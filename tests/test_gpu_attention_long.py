@@ -132,3 +132,33 @@ def test_sdpa_long_fully_masked_rows_are_nan(b):
     assert np.isnan(got[200:240]).all()
     assert np.isfinite(np.delete(got, np.s_[200:240], 0)).all()
     np.testing.assert_array_equal(got[600], read32(b, t[2])[0, 0, 0])  # one visible key: its V
+
+
+@pytest.mark.parametrize("B,H,Lq,copy", [(1, 4, 1100, True), (1, 4, 1, True), (24, 4, 1, False), (24, 4, 150, False),
+                                         (24, 4, 1025, True)])
+def test_rope_of_k_in_a_pass_where_it_is_shared(B, H, Lq, copy):
+    """Fused RoPE takes a rotated copy of K (scratch of the pool) where many
+    query tiles or few heads share the pass, and the same bits come out as
+    from operands rotated beforehand."""
+    from laya_hip.backend import HipBackend
+    b, Lk = HipBackend(0), 1100
+    try:
+        rng = np.random.default_rng(Lq)
+        q, k, v = [b.fromHost(to_host(rng.standard_normal((B, H, n, 64)), "f16")) for n in (Lq, Lk, Lk)]
+        qr, kr = b.rope(q, 10000.0), b.rope(k, 10000.0)
+        b.flush(qr, kr)
+        want = read32(b, b.sdpa(qr, kr, v, None, 0.125))
+        out = b._malloc(B * H * Lq * 64 * 2)
+        st = [F.i64s((H * n * 64, n * 64, 64, 1)) for n in (Lq, Lk)]
+        b.pool_stats()  # (returns the blocks that wait for reuse)
+        b.n.call("trim", "hb_pool_trim", b.ctx)
+        before = b.pool_stats()
+        b.n.call("sdpa", "hb_sdpa", b.ctx, F.HB_F16, b._ptr(q), st[0], b._ptr(k), st[1], b._ptr(v), st[1], 0,
+                 F.i64s((0, 0, 0, 1)), 0, out.ptr, st[0], B, H, Lq, Lk, 64, 0.125, 10000.0, 10000.0)
+        after = b.pool_stats()
+        assert (after["cached_bytes"] - before["cached_bytes"] >= B * H * Lk * 64 * 2) == copy
+        got = np.empty((B, H, Lq, 64), np.float16)
+        b.n.call("read", "hb_download", b.ctx, got.ctypes.data, out.ptr, got.nbytes)
+        np.testing.assert_array_equal(got.astype(np.float32), want)
+    finally:
+        b.destroy()
