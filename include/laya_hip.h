@@ -191,6 +191,12 @@ int hb_linear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintptr_t w, uint
  *  fail.  The arithmetic is the same as with row-major operands, bit for
  *  bit. */
 
+/* The kernel that hb_linear takes for f16 / bf16 operands of 16-byte alignment
+ * on a device of `cus` CUs, as a short name ("ring 64x64", "mfma 128x128",
+ * "arow 192"); K % 8 == 0, `flags` as above.  No GPU call.  For tests that
+ * compare kernels. */
+int hb_linear_kernel(int cus, int64_t ldx, int64_t M, int64_t N, int64_t K, unsigned flags, char* name, size_t cap);
+
 /* The attention block's q / k / v projection fused with its layout glue
  * and RoPE: y = x . w^T for the stacked projection w [3*H*64, K] (no bias,
  * as ModernBERT's attention_bias = false; `bias` must be 0),

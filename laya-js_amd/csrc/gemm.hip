@@ -11,10 +11,13 @@
 //   same LDS C tile) is staged in LDS and written during the first stages of
 //   the block's next tile.  X and Y may be row-major or in panel order
 //   (32-row x 16-column blocks of 1 KB laid out as MFMA operands);
-// - gemm_ring (K % 64 == 0, smaller M): X and W through an LDS ring of K stages
-//   filled by direct loads, one barrier per stage; row-major or panel order;
-// - gemm_mfma (other K below M = 4096): 128 x 128 or 128 x 64 tiles, A and B
-//   double-buffered in LDS, epilogue staged in LDS, 16-byte stores.
+// - gemm_ring (K % 64 == 0, fewer rows or columns): X and W through an LDS ring of
+//   K stages filled by direct loads, one barrier per stage; row-major or panel
+//   order;
+// - gemm_mfma (below M = 4096: other K, and between the two): 128 x 128 or 128 x
+//   64 tiles, A and B double-buffered in LDS, epilogue staged in LDS, 16-byte
+//   stores.
+// linear_kernel (gemm_kernels.h) says which one a call takes.
 // W tiles are 64-wide K stages of 16-byte chunks XOR-swizzled by row so the
 // fragment reads of consecutive rows spread over the LDS banks.  The
 // epilogue adds the bias, rounds once to the storage type, applies GeGLU on
@@ -30,6 +33,7 @@
 //
 // gemm_simt is the f32 path (and the fallback for shapes the MFMA kernel's
 // 16-byte loads cannot take: K or row strides not a multiple of 8).
+#include <cstdio>
 #include <stdexcept>
 #include <type_traits>
 
@@ -305,6 +309,16 @@ extern "C" int hb_linear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintpt
     }
   }
   check_launch("hb_linear");
+  HB_API_END
+}
+
+extern "C" int hb_linear_kernel(int cus, int64_t ldx, int64_t M, int64_t N, int64_t K, unsigned flags, char* name,
+                                size_t cap) {
+  HB_API_BEGIN
+  HB_REQUIRE(cus > 0 && M > 0 && N > 0 && K > 0 && K % 8 == 0 && name && cap > 0, "hb_linear_kernel: bad arguments");
+  std::snprintf(name, cap, "%s", linear_kernel_name(linear_kernel(cus, M, N, K, (flags & HB_X_PANEL) ? K : ldx,
+                                                                  flags & HB_EPI_GEGLU,
+                                                                  flags & (HB_X_PANEL | HB_Y_PANEL))));
   HB_API_END
 }
 

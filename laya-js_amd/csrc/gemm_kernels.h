@@ -1458,42 +1458,66 @@ void launch_ring_t(hipStream_t st, unsigned pan, const uint16_t* x, int64_t ldx,
 // Operands the ring kernel's 32-bit offsets reach.
 inline bool ring_ok(int64_t ldx, int64_t K) { return K % 64 == 0 && K < (1 << 22) && ldx < (1 << 22); }
 
+// The kernels of a linear layer with 16-bit weights (and, the mfma ones, with
+// codes that their loader dequantizes).
+enum class LinearKernel {
+  kRing32x64,     // six stages
+  kRing64x64,     // four stages
+  kRing64x64k,    // five: K chains of 32 and more stages wait for memory
+  kRing64x64x3,   // three, so that three blocks share a CU
+  kRing128x64,
+  kRing128x256,
+  kMfma128x64,
+  kMfma128x128,
+  kArow192,
+  kArow192Tail,   // any K
+  kArow128,
+  kArow128Tail,
+};
+inline bool is_ring(LinearKernel k) { return k <= LinearKernel::kRing128x256; }
+inline const char* linear_kernel_name(LinearKernel k) {
+  static const char* const names[] = {"ring 32x64",  "ring 64x64",   "ring 64x64 long", "ring 64x64 three",
+                                      "ring 128x64", "ring 128x256", "mfma 128x64",     "mfma 128x128",
+                                      "arow 192",    "arow 192 tail", "arow 128",       "arow 128 tail"};
+  return names[(int)k];
+}
+
 // The ring's tile, by how many of each shape the call has (wrows: weight rows;
-// us, f16, back to back; 64 x 64 / 128 x 64 / 64 x 64 with three stages / 128 x
-// 256, and what the kernels before it took):
+// us, f16, back to back; 64 x 64 / 128 x 64 / 64 x 64 with three stages, and the
+// 128-row kernel):
 // - 32 x 64, six stages, while they fit one per CU: with weights that come from
 //   HBM (a model's layers in turn), where the bytes a launch has in flight count,
 //   128 x 2304 x 768 7.9 -> 6.7, 128 x 2304 x 768 GeGLU 8.2 -> 7.0 against 64 x 64;
 // - 64 x 64, four stages, while those fit: 128 x 768 x 768 (24 tiles)
-//   5.8 / 7.4 / 6.3 / 15.0 (9.7), 256 x 2304 x 768 (144) 5.9 / 7.4 / 6.6 / 14.3
-//   (11.5); from K = 2048 five stages, as K chains of 48 stages wait for memory:
-//   512 x 768 x 3072 16.1 -> 13.7 (32.5);
-// - 128 x 64 while those fit: 512 x 3072 x 768 (192) 10.7 / 8.3 / 11.3 / 14.7
-//   (12.1), 768 x 2304 x 768 (216) 8.7 / 8.4 / 9.3 / 15.4 (12.3);
-// - 128 x 256, one round of them that fills more than half the CUs: 2048 x 2304
-//   x 768 (144) 19.4 / 21.9 / 18.7 / 17.6 (21.9), 3072 x 2304 x 768 (216) 24.9 /
-//   28.0 / 25.6 / 19.7 (23.6);
-// - else 64 x 64 with three stages, three blocks per CU: 1024 x 3072 x 768
-//   15.4 / 15.7 / 12.6 / 19.0 (16.4), 4096 x 768 x 768 12.1 / 14.0 / 11.1 / 15.7
-//   (25.6, the large-M kernel).
-template <bool BF16, bool GEGLU>
-void launch_ring(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int64_t ldx, const uint16_t* w,
-                 const uint16_t* bias, const uint16_t* r, int64_t ldr, uint16_t* y, int64_t ldy, int M, int N, int K) {
-  const int64_t wrows = GEGLU ? 2 * (int64_t)N : N;
+//   5.8 / 7.4 / 6.3 (9.7), 256 x 2304 x 768 (144) 5.9 / 7.4 / 6.6 (11.5); from
+//   K = 2048 five stages: 512 x 768 x 3072 16.1 -> 13.7 (32.5);
+// - 128 x 64 while those fit: 512 x 3072 x 768 (192) 10.7 / 8.3 / 11.3 (12.1),
+//   768 x 2304 x 768 (216) 8.7 / 8.4 / 9.3 (12.3);
+// - 64 x 64 with three stages while three fit a CU: 1024 x 3072 x 768 15.4 /
+//   15.7 / 12.6 (16.4), 4096 x 768 x 768 12.1 / 14.0 / 11.1;
+// - 128 x 256, one round of them that fills more than half the CUs, K of 512 to
+//   1536 (beyond that its three stages wait for weights from HBM: 2048 x 2304 x
+//   3072 69 against 58 us) and no GeGLU (whose epilogue costs its single block a
+//   CU more: 2048 x 1152 x 768 21.5 / 19.7): 2048 x 2304 x 768 (144 tiles) 18.3,
+//   the 128-row kernel 20.5; 3072 x 2304 x 768 (216) 20.4, 22.5; with weights
+//   from HBM 23.1 / 20.6 and 23.7 / 23.5;
+// - 64 x 64 with three stages in up to three rounds where the 128-row kernel's
+//   128 x 128 tiles begin a second round (two fit a CU): 4095 x 2304 x 768 30 /
+//   36, 3072 x 3072 x 1024 38 / 44;
+// - else none below M = 4096 (`wide` false): the 128-row kernel reads half as
+//   much LDS per product as a 64 x 64 tile.  1536 x 2304 x 768 18.0 / 16.0 us,
+//   2048 x 2624 x 1024 GeGLU 56.8 / 43.4, 3840 x 4096 x 1024 68.1 / 51.9.
+inline bool ring_tile(int cus, int64_t M, int64_t wrows, int64_t K, bool geglu, bool wide, LinearKernel* tile) {
   auto tiles = [&](int bm, int bn) { return ((M + (int64_t)bm - 1) / bm) * ((wrows + bn - 1) / bn); };
-  const int64_t wide = tiles(128, 256);
-  if (tiles(32, 64) <= cus)
-    launch_ring_t<32, 64, 1, 2, 6, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
-  else if (tiles(64, 64) <= cus && K < 2048)
-    launch_ring_t<64, 64, 2, 2, 4, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
-  else if (tiles(64, 64) <= cus)
-    launch_ring_t<64, 64, 2, 2, 5, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
-  else if (tiles(128, 64) <= cus)
-    launch_ring_t<128, 64, 4, 2, 4, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
-  else if (wide > cus / 2 && wide <= cus)
-    launch_ring_t<128, 256, 4, 4, 3, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
-  else
-    launch_ring_t<64, 64, 2, 2, 3, BF16, GEGLU>(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
+  const int64_t t64 = tiles(64, 64), t256 = tiles(128, 256);
+  if (tiles(32, 64) <= cus) *tile = LinearKernel::kRing32x64;
+  else if (t64 <= cus) *tile = K < 2048 ? LinearKernel::kRing64x64 : LinearKernel::kRing64x64k;
+  else if (tiles(128, 64) <= cus) *tile = LinearKernel::kRing128x64;
+  else if (t64 <= 3 * (int64_t)cus) *tile = LinearKernel::kRing64x64x3;
+  else if (t256 > cus / 2 && t256 <= cus && !geglu && K >= 512 && K <= 1536) *tile = LinearKernel::kRing128x256;
+  else if (wide || (t64 <= 9 * (int64_t)cus && tiles(128, 128) > 2 * (int64_t)cus)) *tile = LinearKernel::kRing64x64x3;
+  else return false;
+  return true;
 }
 
 // From M = 4096, the ring kernel still beats the large-M one where its 256 x 192
@@ -1521,61 +1545,73 @@ inline bool small_panel_path(int64_t M, int64_t N_out, int64_t K, bool geglu, in
 // at); both take panel-order operands.
 inline bool arow_path(int64_t M) { return M >= 4096; }
 
-// Below M = 4096 with K % 64 != 0: 128 x 64 tiles (instead of
-// 128 x 128) where 128 x 128 tiles would leave the GPU short of blocks.
+// 128 x 64 tiles of the 128-row kernel (instead of 128 x 128) where 128 x 128
+// tiles would leave the GPU short of blocks: the K stages of a block run one
+// after another, so a launch with few blocks is bound by that chain.
 // N_out: output columns (GeGLU: value / gate pairs).
 inline bool thin_tiles(int64_t M, int64_t N_out, bool geglu, int cus) {
   const int64_t t128 = ((M + 127) / 128) * ((N_out + (geglu ? 63 : 127)) / (geglu ? 64 : 128));
   return t128 <= cus + cus / 8;
 }
 
+// The kernel a call with 16-bit weights takes.  `ldx`: X's row stride, K in
+// panel order; `panel`: X or Y in panel order, which the 128-row kernel does
+// not take.  Every output keeps its MFMA sequence and epilogue, so the bits do
+// not depend on the choice.
+inline LinearKernel linear_kernel(int cus, int64_t M, int64_t N_out, int64_t K, int64_t ldx, bool geglu, bool panel) {
+  // 128-column tiles of the large-M kernel where N is a multiple of 128 and
+  // not of 192 (N = 1024: 8 whole tiles instead of 5 1/3 of 192 columns)
+  const bool n128 = !geglu && N_out % 192 != 0 && N_out % 128 == 0;
+  const bool ring = ring_ok(ldx, K), large = arow_path(M);
+  LinearKernel tile;
+  if (ring && (!large || ring_beats_arow(M, N_out, K, geglu, n128 ? 128 : 192, cus)) &&
+      ring_tile(cus, M, geglu ? 2 * N_out : N_out, K, geglu, large || panel, &tile))
+    return tile;
+  if (large) {
+    if (K % 64 == 0) return n128 ? LinearKernel::kArow128 : LinearKernel::kArow192;
+    return n128 ? LinearKernel::kArow128Tail : LinearKernel::kArow192Tail;
+  }
+  return thin_tiles(M, N_out, geglu, cus) ? LinearKernel::kMfma128x64 : LinearKernel::kMfma128x128;
+}
+
 template <bool BF16, bool GEGLU, int QB, bool AFF, bool SF32>
 void mfma_dispatch(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int64_t ldx, const uint16_t* w,
                           QW qw, const uint16_t* bias, const uint16_t* r, int64_t ldr, uint16_t* y, int64_t ldy, int M,
                           int N, int K) {
-  // K % 64 == 0: the ring kernel, or from M = 4096 persistent 256 x 192 tiles with
-  // register-resident A rows (hb_qlinear dequantizes a quantized weight once and
-  // calls the 16-bit path).  Other K: the large-M variant with a K tail, below M
-  // = 4096 the 128-row tiles.
+  // (codes are read by the 128-row kernel alone: hb_qlinear dequantizes them
+  // beforehand for the others)
+  HB_REQUIRE(QB == 0 || !arow_path(M), "hb_qlinear: large-M quantized weights are dequantized before the GEMM");
+  const LinearKernel kern = QB == 0 ? linear_kernel(cus, M, N, K, (pan & HB_X_PANEL) ? K : ldx, GEGLU, pan != 0)
+                            : thin_tiles(M, N, GEGLU, cus) ? LinearKernel::kMfma128x64
+                                                           : LinearKernel::kMfma128x128;
   if constexpr (QB == 0) {
-    // 128-column tiles of the large-M kernel where N is a multiple of 128 and
-    // not of 192 (N = 1024: 8 whole tiles instead of 5 1/3 of 192 columns)
-    const bool n128 = !GEGLU && N % 192 != 0 && N % 128 == 0;
-    if (ring_ok((pan & HB_X_PANEL) ? K : ldx, K) && (!arow_path(M) || ring_beats_arow(M, N, K, GEGLU, n128 ? 128 : 192, cus))) {
-      launch_ring<BF16, GEGLU>(st, cus, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
-      return;
+    auto args = [&](auto launch) { launch(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K); };
+    auto arow = [&](auto launch) { launch(st, cus, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K, QK{nullptr, 1, 1}); };
+    switch (kern) {
+      case LinearKernel::kRing32x64: return args(launch_ring_t<32, 64, 1, 2, 6, BF16, GEGLU>);
+      case LinearKernel::kRing64x64: return args(launch_ring_t<64, 64, 2, 2, 4, BF16, GEGLU>);
+      case LinearKernel::kRing64x64k: return args(launch_ring_t<64, 64, 2, 2, 5, BF16, GEGLU>);
+      case LinearKernel::kRing64x64x3: return args(launch_ring_t<64, 64, 2, 2, 3, BF16, GEGLU>);
+      case LinearKernel::kRing128x64: return args(launch_ring_t<128, 64, 4, 2, 4, BF16, GEGLU>);
+      case LinearKernel::kRing128x256:
+        if constexpr (!GEGLU) return args(launch_ring_t<128, 256, 4, 4, 3, BF16, GEGLU>);
+        break;
+      case LinearKernel::kArow192: return arow(launch_arow<192, BF16, GEGLU, false>);
+      case LinearKernel::kArow192Tail: return arow(launch_arow<192, BF16, GEGLU, true>);
+      case LinearKernel::kArow128:
+        if constexpr (!GEGLU) return arow(launch_arow<128, BF16, false, false>);
+        break;
+      case LinearKernel::kArow128Tail:
+        if constexpr (!GEGLU) return arow(launch_arow<128, BF16, false, true>);
+        break;
+      default: break;
     }
-    if (arow_path(M)) {
-      if constexpr (!GEGLU) {
-        if (n128) {
-          if (K % 64 == 0)
-            launch_arow<128, BF16, false, false>(st, cus, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
-          else
-            launch_arow<128, BF16, false, true>(st, cus, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
-          return;
-        }
-      }
-      if (K % 64 == 0)
-        launch_arow<192, BF16, GEGLU, false>(st, cus, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
-      else
-        launch_arow<192, BF16, GEGLU, true>(st, cus, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K);
-      return;
-    }
-  } else {
-    HB_REQUIRE(!arow_path(M), "hb_qlinear: large-M quantized weights are dequantized before the GEMM");
   }
-  {
-    HB_REQUIRE(pan == 0, "hb_linear: panel-order operands on a kernel that does not take them");
-    // Tiles of 128 x 64 (waves of 32 x 64) where 128 x 128 tiles would leave the
-    // GPU short of blocks: the K stages of a block run one after another, so a
-    // launch with few blocks is bound by that chain.  Every output keeps its
-    // MFMA sequence and epilogue, so the bits do not change.
-    if (thin_tiles(M, N, GEGLU, cus)) {
-      launch_mfma<128, 64, 4, 1, BF16, GEGLU, QB, AFF, SF32>(st, x, ldx, w, qw, bias, r, ldr, y, ldy, M, N, K);
-      return;
-    }
+  HB_REQUIRE(pan == 0, "hb_linear: panel-order operands on a kernel that does not take them");
+  if (kern == LinearKernel::kMfma128x64)
+    launch_mfma<128, 64, 4, 1, BF16, GEGLU, QB, AFF, SF32>(st, x, ldx, w, qw, bias, r, ldr, y, ldy, M, N, K);
+  else
     launch_mfma<128, 128, 2, 2, BF16, GEGLU, QB, AFF, SF32>(st, x, ldx, w, qw, bias, r, ldr, y, ldy, M, N, K);
-  }
 }
 
 template <int QB, bool AFF, bool SF32>

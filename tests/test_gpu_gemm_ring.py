@@ -1,8 +1,12 @@
-"""The ring GEMM (16-bit weights, K % 64 == 0): every tile shape at its edges,
-against the oracle at the GEMM bounds (max-rel 2e-3 f16, 8e-3 bf16: the
+"""The GEMM kernels below M = 4096 (16-bit weights): every tile shape of the ring
+kernel at its edges, and the 128-row kernel where it takes a call with K % 64 ==
+0, against the oracle at the GEMM bounds (max-rel 2e-3 f16, 8e-3 bf16: the
 rounding of the stored result, 2^-11 and 2^-8, with room for the f32 sums) and
 bit for bit against the other tiles and the large-M kernel, which run the same
-MFMA steps in the same order."""
+MFMA steps in the same order.  hb_linear_kernel names the kernel each shape is
+here for (on 256 CUs)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -14,10 +18,15 @@ pytestmark = pytest.mark.gpu
 TOL = {"f16": 2e-3, "bf16": 8e-3}
 
 # (M, N, K): one 32 x 64 tile and less; a few with row and column remainders;
-# K shorter than the ring and long; 64 x 64 with four stages and, from K = 2048,
-# five; 128 x 64 tiles; 64 x 64 with three stages; 128 x 256
-SHAPES = [(1, 8, 64), (65, 72, 128), (130, 200, 768), (70, 136, 2112), (520, 1032, 192), (520, 1032, 2112),
-          (900, 1304, 192), (1030, 3000, 64), (2100, 2120, 128), (4100, 768, 256)]
+# K shorter than the ring and long
+SHAPES = [(1, 8, 64, "ring 32x64"), (65, 72, 128, "ring 32x64"), (130, 200, 768, "ring 32x64"),
+          (70, 136, 2112, "ring 32x64"), (520, 1032, 192, "ring 64x64"), (520, 1032, 2112, "ring 64x64 long"),
+          (900, 1304, 192, "ring 128x64"), (1030, 2600, 64, "ring 64x64 three"), (2100, 4104, 64, "ring 64x64 three"),
+          (4100, 768, 256, "ring 64x64 three"), (2100, 2120, 768, "ring 128x256"), (1030, 3000, 64, "mfma 128x64"),
+          (2100, 2120, 128, "mfma 128x128")]
+GEGLU_SHAPES = [(1, 8, 64, "ring 32x64"), (65, 40, 128, "ring 32x64"), (300, 648, 2112, "ring 32x64"),
+                (520, 520, 192, "ring 64x64"), (520, 520, 2112, "ring 64x64 long"), (900, 648, 192, "ring 128x64"),
+                (1030, 1304, 64, "ring 64x64 three"), (1030, 1504, 64, "mfma 128x64"), (2100, 1064, 128, "mfma 128x128")]
 
 
 @pytest.fixture(scope="module")
@@ -26,6 +35,13 @@ def b():
     be = HipBackend(0)
     yield be
     be.destroy()
+
+
+def _takes(b, M, N, K, want, flags=0):
+    """The call's kernel is the one the shape is listed for."""
+    name = ctypes.create_string_buffer(64)
+    b.n.call("kernel", "hb_linear_kernel", b.cus, K, M, N, K, flags, name, len(name))
+    assert name.value.decode() == want
 
 
 def _operands(b, rng, M, N, K, dtype, geglu):
@@ -38,8 +54,9 @@ def _operands(b, rng, M, N, K, dtype, geglu):
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
-@pytest.mark.parametrize("M,N,K", SHAPES)
-def test_ring_tiles(b, M, N, K, dtype):
+@pytest.mark.parametrize("M,N,K,kernel", SHAPES)
+def test_ring_tiles(b, M, N, K, kernel, dtype):
+    _takes(b, M, N, K, kernel)
     print(f"ring M={M} N={N} K={K} {dtype}", flush=True)
     rng = np.random.default_rng(M + N + K)
     (x, w, bias, r), (X, W, B, R) = _operands(b, rng, M, N, K, dtype, False)
@@ -54,9 +71,9 @@ def test_ring_tiles(b, M, N, K, dtype):
         np.testing.assert_array_equal(read32(b, b.linear(xi, W, B))[0], got[i])
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (65, 40, 128), (300, 648, 2112), (520, 520, 192), (900, 648, 192), (1030, 1504, 64),
-                                   (2100, 1064, 128)])
-def test_ring_geglu(b, M, N, K):
+@pytest.mark.parametrize("M,N,K,kernel", GEGLU_SHAPES)
+def test_ring_geglu(b, M, N, K, kernel):
+    _takes(b, M, N, K, kernel, F.HB_EPI_GEGLU)
     """Value and gate columns in one tile, in waves of their own: the bits of
     the separate op on the linear's output; N not a multiple of the tile's
     value columns (but of 8: rows of other lengths take the SIMT kernel, whose
@@ -70,9 +87,12 @@ def test_ring_geglu(b, M, N, K):
     np.testing.assert_array_equal(read32(b, fused), read32(b, want))
 
 
-@pytest.mark.parametrize("M", [100, 700, 1030, 2048])
-def test_ring_bits_equal_large_m(b, M):
+@pytest.mark.parametrize("M,kernel", [(100, "ring 32x64"), (250, "ring 64x64"), (700, "ring 128x64"), (1030, "ring 64x64 three"),
+                                      (2048, "ring 128x256"), (1536, "mfma 128x64"), (4000, "ring 64x64 three")])
+def test_ring_bits_equal_large_m(b, M, kernel):
     """2304 x 768 weights: each tile shape's rows are the large-M kernel's."""
+    _takes(b, M, 2304, 768, kernel)
+    _takes(b, 6144, 2304, 768, "arow 192")
     rng = np.random.default_rng(M)
     (x, w, _, _), (X, W, _, _) = _operands(b, rng, M, 2304, 768, "f16", False)
     big = b.fromHost(to_host(np.resize(x, (6144, 768)), "f16"))

@@ -1,0 +1,36 @@
+"""Which kernel a linear layer with 16-bit weights takes (hb_linear_kernel, no GPU
+call): the lines of the rule, at sizes where both sides were measured on 256 CUs."""
+import ctypes
+
+import pytest
+
+from laya_hip import ffi as F
+
+GEGLU = F.HB_EPI_GEGLU
+
+
+def kernel(M, N, K, flags=0, ldx=None, cus=256):
+    name = ctypes.create_string_buffer(64)
+    n = F.native()
+    n.call("linear_kernel", "hb_linear_kernel", cus, K if ldx is None else ldx, M, N, K, flags, name, len(name))
+    return name.value.decode()
+
+
+@pytest.mark.parametrize("M,N,K,geglu,want", [
+    (1, 768, 768, 0, "ring 32x64"), (93, 2304, 768, 0, "ring 32x64"), (256, 2304, 768, 0, "ring 64x64"),
+    (768, 768, 3072, 0, "ring 64x64 long"), (512, 3072, 768, 0, "ring 128x64"), (512, 1152, 768, 1, "ring 128x64"),
+    (1024, 2304, 768, 0, "ring 64x64 three"), (3840, 768, 768, 0, "ring 64x64 three"),
+    (2048, 2304, 768, 0, "ring 128x256"), (3584, 2304, 768, 0, "ring 128x256"), (2560, 3072, 1024, 0, "ring 128x256"),
+    # the 128-row kernel where the ring's tiles were slower: GeGLU, K = 3072, more than a round
+    (2048, 1152, 768, 1, "mfma 128x64"), (3072, 1152, 768, 1, "mfma 128x128"), (2048, 2304, 3072, 0, "mfma 128x64"),
+    (700, 2624, 1024, 1, "mfma 128x64"), (2048, 2624, 1024, 1, "mfma 128x128"), (3072, 2624, 1024, 1, "mfma 128x128"),
+    (1536, 2304, 768, 0, "mfma 128x64"), (1024, 4096, 1024, 0, "mfma 128x64"), (3840, 4096, 1024, 0, "mfma 128x128"),
+    (3840, 1024, 4096, 0, "mfma 128x64"), (700, 50368, 768, 0, "mfma 128x128"),
+    # its 128 x 128 tiles just over two a CU: the ring's three rounds
+    (3840, 2304, 768, 0, "ring 64x64 three"), (3072, 3072, 1024, 0, "ring 64x64 three"),
+    # other K; from M = 4096
+    (512, 768, 776, 0, "mfma 128x64"), (4096, 2304, 768, 0, "arow 192"), (4096, 768, 768, 0, "ring 64x64 three"),
+    (16384, 1024, 1024, 0, "arow 128"), (4096, 768, 776, 0, "arow 192 tail"),
+])
+def test_the_rule(M, N, K, geglu, want):
+    assert kernel(M, N, K, GEGLU if geglu else 0) == want
