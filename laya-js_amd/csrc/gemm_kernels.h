@@ -1455,7 +1455,8 @@ void launch_ring_t(hipStream_t st, unsigned pan, const uint16_t* x, int64_t ldx,
                                                                   (pan & HB_X_PANEL) ? 1 : 0, (pan & HB_Y_PANEL) ? 1 : 0);
 }
 
-// Operands the ring kernel's 32-bit offsets reach.
+// Operands that the ring kernel's and the large-M kernel's 32-bit offsets reach
+// (the last row of a tile is at most 255 strides away).
 inline bool ring_ok(int64_t ldx, int64_t K) { return K % 64 == 0 && K < (1 << 22) && ldx < (1 << 22); }
 
 // The kernels of a linear layer with 16-bit weights (and, the mfma ones, with
@@ -1470,7 +1471,7 @@ enum class LinearKernel {
   kMfma128x64,
   kMfma128x128,
   kArow192,
-  kArow192Tail,   // any K
+  kArow192Tail,   // any K, 64-bit addresses
   kArow128,
   kArow128Tail,
 };
@@ -1567,8 +1568,9 @@ inline LinearKernel linear_kernel(int cus, int64_t M, int64_t N_out, int64_t K, 
   if (ring && (!large || ring_beats_arow(M, N_out, K, geglu, n128 ? 128 : 192, cus)) &&
       ring_tile(cus, M, geglu ? 2 * N_out : N_out, K, geglu, large || panel, &tile))
     return tile;
-  if (large) {
-    if (K % 64 == 0) return n128 ? LinearKernel::kArow128 : LinearKernel::kArow192;
+  if (large || panel) {
+    // (X rows too far apart for 32-bit offsets: the tail variant's are 64-bit)
+    if (ring) return n128 ? LinearKernel::kArow128 : LinearKernel::kArow192;
     return n128 ? LinearKernel::kArow128Tail : LinearKernel::kArow192Tail;
   }
   return thin_tiles(M, N_out, geglu, cus) ? LinearKernel::kMfma128x64 : LinearKernel::kMfma128x128;

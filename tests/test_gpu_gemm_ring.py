@@ -123,3 +123,23 @@ def test_ring_panel_operands(b, M, N, K, geglu):
     call(xp.ptr, yp.ptr, fl | F.HB_X_PANEL | F.HB_Y_PANEL)
     b.n.call("unpack", "hb_panel_unpack", b.ctx, yp.ptr, yu.ptr, N, M, N)
     np.testing.assert_array_equal(bits(yu.ptr), want)
+
+
+@pytest.mark.parametrize("M,N,K,geglu", [(3, 48, 128, 0), (33, 128, 64, 0), (35, 32, 192, 1)])
+def test_panel_output_of_rows_far_apart(b, M, N, K, geglu):
+    """A row-major x with 2^22 or more elements between its rows (past 32-bit byte
+    offsets within a tile) and y in panel order: the bits of the dense call."""
+    rng = np.random.default_rng(M)
+    _, (X, W, B, _) = _operands(b, rng, M, N, K, "f16", bool(geglu))
+    ldx = 1 << 22
+    far, y, yp, yu = (b._malloc(n) for n in (((M - 1) * ldx + K) * 2, M * N * 2, (M + 31) // 32 * 32 * N * 2, M * N * 2))
+    for i in range(M):
+        b.n.call("copy", "hb_copy", b.ctx, far.ptr + 2 * i * ldx, b._ptr(X) + 2 * i * K, 2 * K)
+    fl = F.HB_EPI_BIAS | (F.HB_EPI_GEGLU if geglu else 0)
+    for x, ld, out, flags in ((b._ptr(X), K, y, fl), (far.ptr, ldx, yp, fl | F.HB_Y_PANEL)):
+        b.n.call("linear", "hb_linear", b.ctx, F.HB_F16, x, ld, b._ptr(W), b._ptr(B), 0, 0, out.ptr, N, M, N, K, flags)
+    b.n.call("unpack", "hb_panel_unpack", b.ctx, yp.ptr, yu.ptr, N, M, N)
+    got = [np.empty(M * N, np.uint16) for _ in range(2)]
+    for g, t in zip(got, (yu, y)):
+        b.n.call("read", "hb_download", b.ctx, g.ctypes.data, t.ptr, g.nbytes)
+    np.testing.assert_array_equal(got[0], got[1])

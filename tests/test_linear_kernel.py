@@ -6,7 +6,7 @@ import pytest
 
 from laya_hip import ffi as F
 
-GEGLU = F.HB_EPI_GEGLU
+GEGLU, XP, YP = F.HB_EPI_GEGLU, F.HB_X_PANEL, F.HB_Y_PANEL
 
 
 def kernel(M, N, K, flags=0, ldx=None, cus=256):
@@ -34,3 +34,20 @@ def kernel(M, N, K, flags=0, ldx=None, cus=256):
 ])
 def test_the_rule(M, N, K, geglu, want):
     assert kernel(M, N, K, GEGLU if geglu else 0) == want
+
+
+def test_panel_order_operands_never_meet_the_kernel_without_them():
+    """Every call that check_panel accepts below M = 4096 takes a kernel that reads
+    and writes panel order, whatever the other operand's row stride."""
+    for K in (64, 768, 1280, 2560):
+        for N in (16, 48, 768, 2304, 8192):
+            for M in (1, 33, 128, 500, 1300, 4000):
+                for geglu in (0, GEGLU):
+                    if 64 * K * (2 if geglu else 1) > 160 * 1024 or -(-N // 32) * -(-M // 128) > 256:
+                        continue
+                    for flags in (XP, YP, XP | YP):
+                        for ldx in (K, (1 << 22) - 8, 1 << 22, 1 << 26):
+                            got = kernel(M, N, K, geglu | flags, ldx)
+                            assert not got.startswith("mfma"), (M, N, K, geglu, flags, ldx, got)
+                            if not flags & XP and ldx >= 1 << 22:  # past 32-bit offsets
+                                assert got.endswith("tail"), (M, N, K, ldx, got)
