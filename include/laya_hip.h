@@ -191,11 +191,13 @@ int hb_linear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintptr_t w, uint
  *  fail.  The arithmetic is the same as with row-major operands, bit for
  *  bit. */
 
-/* The kernel that hb_linear takes for f16 / bf16 operands of 16-byte alignment
- * on a device of `cus` CUs, as a short name ("ring 64x64", "mfma 128x128",
- * "arow 192"); K % 8 == 0, `flags` as above.  No GPU call.  For tests that
+/* The kernel that hb_linear (bits 0) or hb_qlinear (bits 8 or 4) takes for
+ * f16 / bf16 operands of 16-byte alignment on a device of `cus` CUs, as a short
+ * name ("ring 64x64", "mfma 128x128", "arow 192"; "codes ..." where its loader
+ * dequantizes); K % 8 == 0, `flags` as above.  No GPU call.  For tests that
  * compare kernels. */
-int hb_linear_kernel(int cus, int64_t ldx, int64_t M, int64_t N, int64_t K, unsigned flags, char* name, size_t cap);
+int hb_linear_kernel(int cus, int64_t ldx, int64_t M, int64_t N, int64_t K, int bits, unsigned flags, char* name,
+                     size_t cap);
 
 /* The attention block's q / k / v projection fused with its layout glue
  * and RoPE: y = x . w^T for the stacked projection w [3*H*64, K] (no bias,
@@ -220,9 +222,9 @@ int hb_linear_qkv(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintptr_t w, 
  * `zeros` are f16 [N, ceil(K/group)].  Weights dequantize to
  * fl16(q*s + z) (fl16(q*s) when symmetric), exactly what host
  * dequantization uploads, and feed the f16 MFMA with f32 accumulation
- * (K % 64 == 0 or M >= 4096, and large calls below that: once per call into
- * a 16-bit copy taken from the context's pool for the duration of the call;
- * otherwise inside the GEMM kernel's weight loader).
+ * (once per call into a 16-bit copy taken from the context's pool for the
+ * duration of the call, or inside the GEMM kernel's weight loader:
+ * whichever is faster for the shape, the copy always from M = 4096 on).
  * Backend.quantizedLinear (index.ts:257-261) via compose.quantizedLinear
  * (compose.ts:407-414).
  *  dt     dtype of x / y / resid / bias: HB_F16, HB_BF16 or HB_F32.

@@ -26,7 +26,8 @@
 // weights are dequantized to fl16(q*s + z) -- one correctly rounded f16 fma,
 // the value host dequantization would upload -- by one routine (dequant8):
 // once per call into a pooled 16-bit copy that the 16-bit kernels then read
-// (dequant_rows_kernel), or in gemm_mfma's W loader.
+// (dequant_rows_kernel), or in gemm_mfma's W loader (dequantizes_first in
+// gemm_kernels.h says which).
 // Blocks walk the tile grid in an XCD-aware order: the hardware deals block b
 // to XCD b % 8, so each XCD is given a contiguous run of row panels (their A
 // rows and the whole W stay in that XCD's L2).
@@ -312,13 +313,16 @@ extern "C" int hb_linear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintpt
   HB_API_END
 }
 
-extern "C" int hb_linear_kernel(int cus, int64_t ldx, int64_t M, int64_t N, int64_t K, unsigned flags, char* name,
-                                size_t cap) {
+extern "C" int hb_linear_kernel(int cus, int64_t ldx, int64_t M, int64_t N, int64_t K, int bits, unsigned flags,
+                                char* name, size_t cap) {
   HB_API_BEGIN
   HB_REQUIRE(cus > 0 && M > 0 && N > 0 && K > 0 && K % 8 == 0 && name && cap > 0, "hb_linear_kernel: bad arguments");
-  std::snprintf(name, cap, "%s", linear_kernel_name(linear_kernel(cus, M, N, K, (flags & HB_X_PANEL) ? K : ldx,
-                                                                  flags & HB_EPI_GEGLU,
-                                                                  flags & (HB_X_PANEL | HB_Y_PANEL))));
+  const bool geglu = flags & HB_EPI_GEGLU;
+  const int64_t ld = (flags & HB_X_PANEL) ? K : ldx;
+  const bool codes = bits != 0 && !dequantizes_first(cus, M, N, K, ld, geglu);
+  const LinearKernel k = codes ? code_kernel(cus, M, N, geglu)
+                               : linear_kernel(cus, M, N, K, ld, geglu, flags & (HB_X_PANEL | HB_Y_PANEL));
+  std::snprintf(name, cap, "%s%s", codes ? "codes " : "", linear_kernel_name(k));
   HB_API_END
 }
 
@@ -414,23 +418,17 @@ extern "C" int hb_qlinear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintp
     const uint16_t* Rp = (const uint16_t*)r;
     uint16_t* Yp = (uint16_t*)y;
     int m = (int)M, n = (int)N, k = (int)K;
-    const int cus0 = cu_count(ctx);
+    const int cus = cu_count(ctx);
     const int64_t rows = geglu ? 2 * N : N;
     CallScratch held(ctx);
-    bool dequant = arow_path(M) || ring_ok(ldx, K) || (M >= 1024 && !thin_tiles(M, N, geglu, cus0));
+    bool dequant = dequantizes_first(cus, M, N, K, (pan & HB_X_PANEL) ? K : ldx, geglu);
     if (dequant && !held.take((size_t)(rows * K * 2))) {
       // no memory for the copy: gemm_mfma's loader dequantizes without one
       HB_REQUIRE(!arow_path(M), "hb_qlinear: out of device memory for the dequantized weight");
       dequant = false;
     }
     if (dequant) {
-      // The weight is dequantized once into a pooled 16-bit copy and the 16-bit
-      // GEMM runs on it: one bandwidth-bound pass over the weight (4-6 us)
-      // instead of the same work in every row tile's loader (M = 512, q4, the
-      // pass included: 1152 x 768 GeGLU 20.7 -> 12.5, 768 x 1152 18.8 -> 11 us).
-      // gemm_mfma dequantizes in its loader where it has few blocks.
       uint16_t* wd = (uint16_t*)held.p;
-      const int cus = cu_count(ctx);
       if (bits == 8 && mode == 0) launch_dequant_rows<8, false>(st, cus, dt, q, wd, rows, k);
       else if (bits == 8) launch_dequant_rows<8, true>(st, cus, dt, q, wd, rows, k);
       else if (mode == 0) launch_dequant_rows<4, false>(st, cus, dt, q, wd, rows, k);
@@ -438,10 +436,10 @@ extern "C" int hb_qlinear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintp
       check_launch("hb_qlinear (dequantize)");
       QW none{nullptr, nullptr, nullptr, 0, 1};
       mfma_dtype<0, false, false>(dt, geglu, st, cus, pan, X, ldx, wd, none, Bp, Rp, ldr, Yp, ldy, m, n, k);
-    } else if (bits == 8 && mode == 0) mfma_dtype<8, false, false>(dt, geglu, st, cu_count(ctx), pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
-    else if (bits == 8) mfma_dtype<8, true, false>(dt, geglu, st, cu_count(ctx), pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
-    else if (mode == 0) mfma_dtype<4, false, false>(dt, geglu, st, cu_count(ctx), pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
-    else mfma_dtype<4, true, false>(dt, geglu, st, cu_count(ctx), pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
+    } else if (bits == 8 && mode == 0) mfma_dtype<8, false, false>(dt, geglu, st, cus, pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
+    else if (bits == 8) mfma_dtype<8, true, false>(dt, geglu, st, cus, pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
+    else if (mode == 0) mfma_dtype<4, false, false>(dt, geglu, st, cus, pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
+    else mfma_dtype<4, true, false>(dt, geglu, st, cus, pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
   } else {
     QWs q{(const uint8_t*)qw, (const void*)scales, (const void*)zeros, HB_F16, G, group, bits, mode};
     dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));

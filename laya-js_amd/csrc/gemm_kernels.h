@@ -1555,6 +1555,11 @@ inline bool thin_tiles(int64_t M, int64_t N_out, bool geglu, int cus) {
   return t128 <= cus + cus / 8;
 }
 
+// The 128-row kernel, which reads codes too.
+inline LinearKernel code_kernel(int cus, int64_t M, int64_t N_out, bool geglu) {
+  return thin_tiles(M, N_out, geglu, cus) ? LinearKernel::kMfma128x64 : LinearKernel::kMfma128x128;
+}
+
 // The kernel a call with 16-bit weights takes.  `ldx`: X's row stride, K in
 // panel order; `panel`: X or Y in panel order, which the 128-row kernel does
 // not take.  Every output keeps its MFMA sequence and epilogue, so the bits do
@@ -1573,7 +1578,25 @@ inline LinearKernel linear_kernel(int cus, int64_t M, int64_t N_out, int64_t K, 
     if (ring) return n128 ? LinearKernel::kArow128 : LinearKernel::kArow192;
     return n128 ? LinearKernel::kArow128Tail : LinearKernel::kArow192Tail;
   }
-  return thin_tiles(M, N_out, geglu, cus) ? LinearKernel::kMfma128x64 : LinearKernel::kMfma128x128;
+  return code_kernel(cus, M, N_out, geglu);
+}
+
+// Whether a quantized weight is dequantized once per call, into a 16-bit copy
+// for the kernel above, instead of in the 128-row kernel's loader in every row
+// tile.  The pass costs a launch and its traffic (5 bytes a weight and more, 1
+// us per million weights once they leave the caches); the loader about 0.6 us
+// a K stage over the ring, whatever the width while its tiles run side by
+// side.  So the ring takes the call where the weight is small against its K
+// chain.  us, pass + ring / loader, q8 to f16: 128 x 2304 x 768 12.5 / 13.9, 512
+// x 768 x 1152 11 / 18.8, 128 x 768 x 3072 19.8 / 41, 256 x 5248 x 1024 15.8 /
+// 17.6; 768 x 48 x 64 6.4 / 5.3, 256 x 16384 x 768 30.8 / 18.8, 1 x 50368 x 768
+// 40 / 25, 1 x 256000 x 1024 261 / 116.  From M = 1024, where the 128-row kernel
+// would run 128 x 128 tiles, its loader repeats the work too often (3072 x 2304
+// x 768 23.9 / 27.8).
+inline bool dequantizes_first(int cus, int64_t M, int64_t N_out, int64_t K, int64_t ldx, bool geglu) {
+  if (arow_path(M) || (M >= 1024 && !thin_tiles(M, N_out, geglu, cus))) return true;
+  return is_ring(linear_kernel(cus, M, N_out, K, ldx, geglu, false)) &&
+         (geglu ? 2 : 1) * N_out * K <= (K / 64 - 4) * 500000;
 }
 
 template <bool BF16, bool GEGLU, int QB, bool AFF, bool SF32>
@@ -1584,8 +1607,7 @@ void mfma_dispatch(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int
   // beforehand for the others)
   HB_REQUIRE(QB == 0 || !arow_path(M), "hb_qlinear: large-M quantized weights are dequantized before the GEMM");
   const LinearKernel kern = QB == 0 ? linear_kernel(cus, M, N, K, (pan & HB_X_PANEL) ? K : ldx, GEGLU, pan != 0)
-                            : thin_tiles(M, N, GEGLU, cus) ? LinearKernel::kMfma128x64
-                                                           : LinearKernel::kMfma128x128;
+                                    : code_kernel(cus, M, N, GEGLU);
   if constexpr (QB == 0) {
     auto args = [&](auto launch) { launch(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K); };
     auto arow = [&](auto launch) { launch(st, cus, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K, QK{nullptr, 1, 1}); };

@@ -57,7 +57,7 @@ SYMBOLS: dict[str, tuple] = {
     "hb_graph_launch": (I, [U, U]),
     "hb_graph_destroy": (I, [U, U]),
     "hb_linear": (I, [U, I, U, I64, U, U, U, I64, U, I64, I64, I64, I64, C.c_uint]),
-    "hb_linear_kernel": (I, [I, I64, I64, I64, I64, C.c_uint, C.c_char_p, C.c_size_t]),
+    "hb_linear_kernel": (I, [I, I64, I64, I64, I64, I, C.c_uint, C.c_char_p, C.c_size_t]),
     "hb_linear_qkv": (I, [U, I, U, I64, U, U, U, I64, I64, I64, I64, D, C.c_uint]),
     "hb_qlinear": (I, [U, I, U, I64, U, U, U, U, U, I64, U, I64, I64, I64, I64, I, I, I, C.c_uint]),
     "hb_qgather": (I, [U, U, U, U, I64, I64, I, I, I, U, I64, I, U]),

@@ -40,7 +40,7 @@ def b():
 def _takes(b, M, N, K, want, flags=0):
     """The call's kernel is the one the shape is listed for."""
     name = ctypes.create_string_buffer(64)
-    b.n.call("kernel", "hb_linear_kernel", b.cus, K, M, N, K, flags, name, len(name))
+    b.n.call("kernel", "hb_linear_kernel", b.cus, K, M, N, K, 0, flags, name, len(name))
     assert name.value.decode() == want
 
 

@@ -1,5 +1,4 @@
-"""Which kernel a linear layer with 16-bit weights takes (hb_linear_kernel, no GPU
-call): the lines of the rule, at sizes where both sides were measured on 256 CUs."""
+"""Which kernel a 16-bit linear layer takes (hb_linear_kernel, no GPU call): the lines of the rule, at sizes where both sides were measured on 256 CUs."""
 import ctypes
 
 import pytest
@@ -9,10 +8,10 @@ from laya_hip import ffi as F
 GEGLU, XP, YP = F.HB_EPI_GEGLU, F.HB_X_PANEL, F.HB_Y_PANEL
 
 
-def kernel(M, N, K, flags=0, ldx=None, cus=256):
+def kernel(M, N, K, flags=0, ldx=None, cus=256, bits=0):
     name = ctypes.create_string_buffer(64)
     n = F.native()
-    n.call("linear_kernel", "hb_linear_kernel", cus, K if ldx is None else ldx, M, N, K, flags, name, len(name))
+    n.call("linear_kernel", "hb_linear_kernel", cus, K if ldx is None else ldx, M, N, K, bits, flags, name, len(name))
     return name.value.decode()
 
 
@@ -51,3 +50,19 @@ def test_panel_order_operands_never_meet_the_kernel_without_them():
                             assert not got.startswith("mfma"), (M, N, K, geglu, flags, ldx, got)
                             if not flags & XP and ldx >= 1 << 22:  # past 32-bit offsets
                                 assert got.endswith("tail"), (M, N, K, ldx, got)
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("M,N,K,geglu,want", [
+    (1, 768, 768, 0, "ring 32x64"), (128, 2304, 768, 0, "ring 32x64"), (512, 768, 1152, 0, "ring 32x64"),
+    (512, 1152, 768, 1, "ring 128x64"), (256, 2624, 1024, 1, "ring 128x64"), (1024, 3072, 1024, 0, "ring 64x64 three"),
+    (3072, 2304, 768, 0, "ring 128x256"), (3072, 2624, 1024, 1, "mfma 128x128"), (16384, 2304, 768, 0, "arow 192"),
+    # a short K chain, or a weight that is wide against it: the loader was faster
+    (1, 48, 64, 0, "codes mfma 128x64"), (4000, 48, 64, 0, "codes mfma 128x64"), (256, 16384, 768, 0, "codes mfma 128x64"),
+    (1, 50368, 768, 0, "codes mfma 128x128"), (33, 256000, 1024, 0, "codes mfma 128x128"),
+    # where the 16-bit call takes the 128-row kernel on few tiles; other K
+    (1536, 2304, 768, 0, "codes mfma 128x64"), (700, 2624, 1024, 1, "codes mfma 128x64"),
+    (2048, 1152, 768, 1, "codes mfma 128x64"), (512, 768, 776, 0, "codes mfma 128x64"),
+])
+def test_where_codes_are_dequantized(M, N, K, geglu, want, bits):
+    assert kernel(M, N, K, GEGLU if geglu else 0, bits=bits) == want
