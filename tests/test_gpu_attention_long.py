@@ -162,3 +162,32 @@ def test_rope_of_k_in_a_pass_where_it_is_shared(B, H, Lq, copy):
         np.testing.assert_array_equal(got.astype(np.float32), want)
     finally:
         b.destroy()
+
+
+@pytest.mark.parametrize("Lq,Lk", [(1, 64), (1, 200), (15, 63), (16, 64), (17, 130), (100, 333), (128, 65), (130, 70),
+                                   (300, 129)])
+def test_mask_classes(b, Lq, Lk):
+    """hb_sdpa_mask_info: one byte per 16 queries x 64 keys, 0 nothing visible,
+    1 everything, 2 mixed or past the last key; groups without queries are 0."""
+    B = 2
+    rng = np.random.default_rng(Lq * 7 + Lk)
+    nqt, nkt = -(-Lq // 128), -(-Lk // 64)
+    for per_query in (True, False):
+        m = np.ones((B, Lq if per_query else 1, Lk), np.uint8)
+        m[1] = rng.random(m[1].shape) < 0.5
+        m[0, :, Lk // 2:] = 0
+        M = b.fromHost(HostTensor("bool", m.shape, m))
+        info = b._malloc(B * nqt * nkt * 8)
+        ms = F.i64s((m.shape[1] * Lk, 0, Lk if per_query else 0, 1))
+        b.n.call("fill", "hb_fill", b.ctx, info.ptr, 77, B * nqt * nkt * 8)
+        b.n.call("info", "hb_sdpa_mask_info", b.ctx, b._ptr(M), ms, B, Lq, Lk, info.ptr)
+        got = np.empty((B, nqt, nkt, 8), np.uint8)
+        b.n.call("read", "hb_download", b.ctx, got.ctypes.data, info.ptr, got.nbytes)
+        want = np.zeros_like(got)
+        full = np.broadcast_to(m, (B, Lq, Lk))
+        for i in range(B):
+            for q in range(0, Lq, 16):
+                for k in range(0, Lk, 64):
+                    t = full[i, q:q + 16, k:k + 64]
+                    want[i, q // 128, k // 64, q // 16 % 8] = 0 if not t.any() else 1 if t.all() and k + 64 <= Lk else 2
+        np.testing.assert_array_equal(got, want)
