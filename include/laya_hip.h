@@ -129,6 +129,12 @@ int hb_free(uintptr_t ctx, uintptr_t ptr);
 int hb_pool_stats(uintptr_t ctx, uint64_t* live_bytes, uint64_t* cached_bytes, uint64_t* live_blocks);
 /* Returns cached blocks to the driver (after a stream sync). */
 int hb_pool_trim(uintptr_t ctx);
+/* For tests: until it is called with 0, every allocation of this context (also
+ * those that a cached block would serve) fails as if the driver had returned
+ * the HIP error code `error` (2: out of memory).  Ops that take scratch for
+ * the duration of a call have another path without it; only out of memory sends
+ * them there. */
+int hb_fail_allocs(uintptr_t ctx, int error);
 
 /* Copies `bytes` from host memory into device memory.  The host buffer is
  * copied into pinned staging before the call returns, so the caller may

@@ -51,6 +51,7 @@ struct Context {
   std::vector<void*> held;
   std::vector<void*> call_scratch;  // live blocks that earlier calls of the recording used and later ones may
   std::map<void*, std::vector<void*>> graph_held;  // hipGraphExec_t -> held blocks
+  hipError_t fail_alloc = hipSuccess;  // hb_fail_allocs: what allocations report instead of being made
 };
 
 static size_t size_class(size_t bytes) {
@@ -89,9 +90,22 @@ struct OutOfMemory : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
 
+// A failed allocation: OutOfMemory only where the device is out of memory, so
+// that a caller with another path takes it then and not after some other error
+// (an earlier launch's, say), which must reach the host.
+[[noreturn]] static void throw_alloc(hipError_t e, size_t bytes, const char* when) {
+  const std::string what = std::to_string(bytes) + " bytes" + when + ": " + hipGetErrorString(e);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();  // not the launches' that follow
+    throw OutOfMemory("hb_alloc: out of device memory for " + what);
+  }
+  throw std::runtime_error("hb_alloc: " + what);
+}
+
 void* pool_alloc(uintptr_t ctx, size_t bytes) {
   Context* c = C(ctx);
   size_t sc = size_class(bytes);
+  if (c->fail_alloc != hipSuccess) throw_alloc(c->fail_alloc, bytes, "");
   auto it = c->free_list.find(sc);
   void* p = nullptr;
   if (it != c->free_list.end() && !it->second.empty()) {
@@ -102,8 +116,7 @@ void* pool_alloc(uintptr_t ctx, size_t bytes) {
     require_current(c);
     hipError_t e = hipMalloc(&p, sc);
     if (e != hipSuccess && c->capturing)  // the retry below would synchronize the recording stream
-      throw OutOfMemory("hb_alloc: out of device memory for " + std::to_string(bytes) +
-                        " bytes while recording a graph");
+      throw_alloc(e, bytes, " while recording a graph");
     if (e != hipSuccess) {
       // release the cache once and retry before failing
       HB_CHECK_HIP(hipStreamSynchronize(c->stream));
@@ -113,9 +126,7 @@ void* pool_alloc(uintptr_t ctx, size_t bytes) {
       c->cached_bytes = 0;
       (void)hipGetLastError();
       e = hipMalloc(&p, sc);
-      if (e != hipSuccess)
-        throw OutOfMemory("hb_alloc: out of device memory for " + std::to_string(bytes) + " bytes: " +
-                          hipGetErrorString(e));
+      if (e != hipSuccess) throw_alloc(e, bytes, "");
     }
   }
   c->live[p] = sc;
@@ -144,7 +155,6 @@ bool CallScratch::take(size_t bytes) {
       p = pool_alloc(ctx, bytes);
       return true;
     } catch (const OutOfMemory&) {
-      (void)hipGetLastError();  // not the launches' that follow
       if (have == 0) return false;
     }
   }
@@ -349,6 +359,12 @@ int hb_pool_trim(uintptr_t ctx) {
     for (void* p : kv.second) HB_CHECK_HIP(hipFree(p));
   c->free_list.clear();
   c->cached_bytes = 0;
+  HB_API_END
+}
+
+int hb_fail_allocs(uintptr_t ctx, int error) {
+  HB_API_BEGIN
+  C(ctx)->fail_alloc = (hipError_t)error;
   HB_API_END
 }
 

@@ -43,6 +43,7 @@ SYMBOLS: dict[str, tuple] = {
     "hb_free": (I, [U, U]),
     "hb_pool_stats": (I, [U, PU64, PU64, PU64]),
     "hb_pool_trim": (I, [U]),
+    "hb_fail_allocs": (I, [U, I]),
     "hb_upload": (I, [U, U, P, C.c_size_t]),
     "hb_download": (I, [U, P, U, C.c_size_t]),
     "hb_copy": (I, [U, U, U, C.c_size_t]),
