@@ -5,12 +5,10 @@ rounding of the stored result, 2^-11 and 2^-8, with room for the f32 sums) and
 bit for bit against the other tiles and the large-M kernel, which run the same
 MFMA steps in the same order.  hb_linear_kernel names the kernel each shape is
 here for (on 256 CUs)."""
-import ctypes
-
 import numpy as np
 import pytest
 
-from gpu_util import max_rel, read32, rounded, to_host
+from gpu_util import linear_kernel, max_rel, read32, rounded, to_host
 from laya_hip import ffi as F
 from oracle import cpu_ref as cr
 
@@ -37,13 +35,6 @@ def b():
     be.destroy()
 
 
-def _takes(b, M, N, K, want, flags=0):
-    """The call's kernel is the one the shape is listed for."""
-    name = ctypes.create_string_buffer(64)
-    b.n.call("kernel", "hb_linear_kernel", b.cus, K, M, N, K, 0, flags, name, len(name))
-    assert name.value.decode() == want
-
-
 def _operands(b, rng, M, N, K, dtype, geglu):
     rows = 2 * N if geglu else N
     x = rounded(rng.standard_normal((M, K)), dtype)
@@ -56,7 +47,7 @@ def _operands(b, rng, M, N, K, dtype, geglu):
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("M,N,K,kernel", SHAPES)
 def test_ring_tiles(b, M, N, K, kernel, dtype):
-    _takes(b, M, N, K, kernel)
+    assert linear_kernel(b, M, N, K) == kernel
     print(f"ring M={M} N={N} K={K} {dtype}", flush=True)
     rng = np.random.default_rng(M + N + K)
     (x, w, bias, r), (X, W, B, R) = _operands(b, rng, M, N, K, dtype, False)
@@ -73,7 +64,7 @@ def test_ring_tiles(b, M, N, K, kernel, dtype):
 
 @pytest.mark.parametrize("M,N,K,kernel", GEGLU_SHAPES)
 def test_ring_geglu(b, M, N, K, kernel):
-    _takes(b, M, N, K, kernel, F.HB_EPI_GEGLU)
+    assert linear_kernel(b, M, N, K, geglu=True) == kernel
     """Value and gate columns in one tile, in waves of their own: the bits of
     the separate op on the linear's output; N not a multiple of the tile's
     value columns (but of 8: rows of other lengths take the SIMT kernel, whose
@@ -91,8 +82,8 @@ def test_ring_geglu(b, M, N, K, kernel):
                                       (2048, "ring 128x256"), (1536, "mfma 128x64"), (4000, "ring 64x64 three")])
 def test_ring_bits_equal_large_m(b, M, kernel):
     """2304 x 768 weights: each tile shape's rows are the large-M kernel's."""
-    _takes(b, M, 2304, 768, kernel)
-    _takes(b, 6144, 2304, 768, "arow 192")
+    assert linear_kernel(b, M, 2304, 768) == kernel
+    assert linear_kernel(b, 6144, 2304, 768) == "arow 192"
     rng = np.random.default_rng(M)
     (x, w, _, _), (X, W, _, _) = _operands(b, rng, M, 2304, 768, "f16", False)
     big = b.fromHost(to_host(np.resize(x, (6144, 768)), "f16"))

@@ -2,8 +2,8 @@
 hb_graph_*): replays give the eager forward's bits.  Each replay is followed
 by eager work on the same backend (an eager encode, which reuses blocks of
 the pool) and a read that synchronizes; every replay is checked.  The shapes
-take both GEMM kernels: the small-M one, and at M = 4096 rows the large-M one
-with panel-order operands from the LayerNorm, attention and GeGLU kernels.  New token
+take the ring GEMM and, at M = 16384 rows, the large-M one with panel-order
+operands from the LayerNorm, attention and GeGLU kernels.  New token
 ids, and then a new padding pattern in the attention masks, written in place
 into the recorded inputs (HipBackend.write) give the eager result for those
 inputs: every replay re-summarises the masks it reads.  Destroying the graph returns its blocks: the pool's live block count
@@ -11,6 +11,7 @@ comes back to where it was before the recording."""
 import numpy as np
 import pytest
 
+from gpu_util import linear_kernel
 from laya_hip import ffi as F
 from laya_hip.host import HostTensor
 from laya_hip.modernbert import attentionMasks, loadModernBert, parseModernBertConfig
@@ -50,8 +51,11 @@ def _bits(b, t):
     return np.asarray(b.read(t).data).view(np.uint16).copy()
 
 
-@pytest.mark.parametrize("B,T", [(1, 128), (2, 96), (8, 512)])  # M = 4096: the large-M GEMM, panel operands
+@pytest.mark.parametrize("B,T", [(1, 128), (2, 96), (8, 512), (32, 512)])  # from M = 4096 on: panel operands
 def test_recorded_encoder_replays(b, B, T):
+    H, I = CFG["hidden_size"], CFG["intermediate_size"]
+    kernels = [linear_kernel(b, B * T, *s).split()[0] for s in ((3 * H, H), (H, H), (I, H, True), (H, I))]
+    assert kernels[0] == ("arow" if B * T >= 16384 else "ring")
     rng = np.random.default_rng(B * 100 + T)
     W = _weights(rng)
     enc = loadModernBert(b, parseModernBertConfig(CFG),
@@ -121,7 +125,8 @@ def test_recorded_quantized_linear_replays(b):
     from laya_hip.host import HostQuantized, pack_quantized
     from oracle import cpu_ref as cr
     rng = np.random.default_rng(9)
-    N, K, M = 768, 768, 4096
+    N, K, M = 2304, 768, 4096
+    assert linear_kernel(b, M, N, K, bits=4) == "arow 192"
     w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
     q, s, z = cr.quantize_matrix(w, N, K, 4, 64, refine=False)
     h = HostQuantized((N, K), 4, 64, "affine", pack_quantized(q, 4), HostTensor("f16", s.shape, s.view(np.float16)),

@@ -10,7 +10,7 @@ dequantization uploads (backend-webgpu/test/quantized.test.ts:107-160)."""
 import numpy as np
 import pytest
 
-from gpu_util import max_rel, read32, rounded, to_host
+from gpu_util import large_m_rows, linear_kernel, max_rel, read32, rounded, to_host
 from laya_hip.host import HostQuantized, HostTensor, QuantizedLinearOptions, pack_quantized
 from oracle import cpu_ref as cr
 
@@ -164,16 +164,17 @@ def test_qlinear_config2(b, name, M, bits):
 
 
 @pytest.mark.parametrize("bits", [8, 4])
-@pytest.mark.parametrize("M", [512, 2048, 4160])
+@pytest.mark.parametrize("M", [512, 1536, 2048, 4160, 6200])
 def test_qlinear_bf16(b, M, bits):
     """Quantized weights with bf16 activations: the dequantized weight is
     rounded once to bf16 (quant.ts:189-243, dequantRows then the compute
-    dtype) on every path -- M = 512 and M = 2048 (128 x 64 tiles, the loader
-    dequantizing each stage) and M = 4160 (dequantized once, then the
-    large-M kernel with a partial row tile) -- against the oracle's
-    dequantize-then-linear in bf16, max-rel <= 1e-2."""
+    dtype) on every path -- M = 1536 (128 x 64 tiles, the loader dequantizing
+    each stage), M = 512, 2048 and 4160 (dequantized once, then the ring kernel)
+    and M = 6200 (then the large-M kernel with a partial row tile) -- against the
+    oracle's dequantize-then-linear in bf16, max-rel <= 1e-2."""
     from laya_hip import compose as C
     N, K = SHAPES["Wqkv"]
+    assert linear_kernel(b, M, N, K, bits=bits).split()[0] == {1536: "codes", 6200: "arow"}.get(M, "ring")
     rng = np.random.default_rng(7 * M + bits)
     h, q, sf, zf = _quantized(rng, N, K, bits)
     x = rounded(rng.standard_normal((M, K)), "bf16")
@@ -190,11 +191,10 @@ def test_qlinear_bf16(b, M, bits):
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
-def test_quantized_small_m_slab_bits_equal_large_m(b, dtype):
-    """Quantized weights on the small-M slab kernel (the slab's codes, scales
-    and zeros fetched to LDS and dequantized once into the f16 slab): against
-    the oracle's dequantize-then-linear (max-rel <= 1e-2), and bit for bit
-    against the same rows inside a 4096-row input, which the large-M kernel
+def test_quantized_small_m_bits_equal_large_m(b, dtype):
+    """Quantized weights in calls of few rows (dequantized once, then the ring
+    kernel): against the oracle's dequantize-then-linear (max-rel <= 1e-2), and
+    bit for bit against the same rows inside a call that the large-M kernel
     computes with the same dequantization and k16 order.  Shapes: attn Wo and
     mlp Wo (K = 1152) with residuals, Wi + GeGLU, a ragged output width with
     K = 576; q8 symmetric and q4 affine; groups of 64 and 32."""
@@ -203,7 +203,7 @@ def test_quantized_small_m_slab_bits_equal_large_m(b, dtype):
     cases = [(128, 768, 768, False, 8, 64, True), (512, 768, 1152, False, 4, 64, True),
              (77, 2304, 768, True, 4, 32, False), (200, 784, 576, False, 8, 32, False)]
     for (M, N2, K, geglu, bits, g, resid) in cases:
-        print(f"quantized slab M={M} N={N2} K={K} geglu={geglu} q{bits} g{g} resid={resid} {dtype}", flush=True)
+        print(f"quantized small M={M} N={N2} K={K} geglu={geglu} q{bits} g{g} resid={resid} {dtype}", flush=True)
         h, q, sf, zf = _quantized(rng, N2, K, bits, g)
         Q = C.upload_quantized(b, h, dtype)
         assert Q.native
@@ -228,34 +228,40 @@ def test_quantized_small_m_slab_bits_equal_large_m(b, dtype):
         ref = r + rounded(ref, dtype) if resid else ref
         err = max_rel(got, ref)
         assert err <= 1e-2, f"M={M} N={N2} K={K} q{bits}: max-rel {err:.2e}"
-        xb = np.concatenate([x, rounded(rng.standard_normal((4096 - M, K)), dtype)])
-        rb = np.concatenate([r, rounded(rng.standard_normal((4096 - M, N)), dtype)])
-        big, _ = run(xb, rb)
+        assert linear_kernel(b, M, N, K, geglu, bits).startswith("ring")
+        ML = large_m_rows(b, N, K, geglu)
+        big, _ = run(np.resize(x, (ML, K)), np.resize(r, (ML, N)))
         np.testing.assert_array_equal(out, big[:M])
         C.dispose_quantized(b, Q)
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_quantized_mid_m_bits_equal_large_m(b, dtype):
-    """Between M = 1024 and 4096 a quantized linear on 128 x 64 tiles
-    dequantizes each W stage in its loader (Wqkv at M = 2048, attn Wo and
-    mlp Wo); Wqkv at M = 3072 runs 128 x 128 tiles on the weight dequantized
-    once into a 16-bit copy.  Every path gives a row the same bits: the rows
-    of an M-row call equal the same rows inside a 4096-row call, which the
-    large-M kernel computes on the weight dequantized once.  Each call is
-    also checked against the oracle's dequantize-then-linear (max-rel <=
-    1e-2).  q8 symmetric and q4 affine, residuals, a ragged M."""
+    """Between M = 1024 and 4096 a quantized linear dequantizes each W stage in
+    the loader of the 128-row kernel, or the whole weight once for the ring or
+    the 128 x 128 tiles.  Every path gives a row the same bits: the rows of an
+    M-row call equal the same rows inside a call of the large-M kernel, on the
+    weight dequantized once.  Each call is also checked against the oracle's
+    dequantize-then-linear (max-rel <= 1e-2).  q8 symmetric and q4 affine,
+    residuals, a ragged M, and K % 64 != 0 (the loader at every M below 4096 of
+    few tiles) over many stages."""
     from laya_hip import compose as C
     rng = np.random.default_rng(43)
-    cases = [(2048, 2304, 768, 8, False), (3072, 2304, 768, 4, False), (2048, 768, 768, 4, True),
-             (1024, 768, 1152, 8, False), (2000, 768, 768, 8, True)]
-    for (M, N, K, bits, resid) in cases:
+    cases = [(1536, 2304, 768, 8, False, "codes mfma 128x64"), (2048, 2304, 768, 8, False, "ring 128x256"),
+             (3072, 2304, 768, 4, False, "ring 128x256"), (2048, 768, 768, 4, True, "ring 128x64"),
+             (1024, 768, 1152, 8, False, "ring 64x64"), (2000, 768, 768, 8, True, "ring 128x64"),
+             (2500, 5248, 256, 4, True, "mfma 128x128"), (700, 2304, 776, 8, True, "codes mfma 128x64"),
+             (130, 768, 1160, 4, True, "codes mfma 128x64"), (900, 5248, 200, 4, False, "codes mfma 128x128")]
+    for (M, N, K, bits, resid, kernel) in cases:
+        assert linear_kernel(b, M, N, K, False, bits) == kernel
+        ML = large_m_rows(b, N, K)
         print(f"quantized mid-M M={M} N={N} K={K} q{bits} resid={resid} {dtype}", flush=True)
-        h, q, sf, zf = _quantized(rng, N, K, bits)
+        g = 64 if K % 64 == 0 else 8
+        h, q, sf, zf = _quantized(rng, N, K, bits, g)
         Q = C.upload_quantized(b, h, dtype)
         assert Q.native
-        x = rounded(rng.standard_normal((4096, K)), dtype)
-        r = rounded(rng.standard_normal((4096, N)), dtype)
+        x = np.resize(rounded(rng.standard_normal((4096, K)), dtype), (ML, K))
+        r = np.resize(rounded(rng.standard_normal((4096, N)), dtype), (ML, N))
 
         def run(xs, rs):
             X, R = b.fromHost(to_host(xs, dtype)), b.fromHost(to_host(rs, dtype))
@@ -270,11 +276,42 @@ def test_quantized_mid_m_bits_equal_large_m(b, dtype):
         (small, got), (big, _) = run(x[:M], r[:M]), run(x, r)
         np.testing.assert_array_equal(small, big[:M])
         rows = _rows(M, rng)
-        lin = cr.quantized_linear(x[rows], q, sf, zf, 64, dtype=dtype)
+        lin = cr.quantized_linear(x[rows], q, sf, zf, g, dtype=dtype)
         ref = r[rows] + rounded(lin, dtype) if resid else lin
         err = max_rel(got[rows], ref)
         assert err <= 1e-2, f"M={M} N={N} K={K} q{bits}: max-rel {err:.2e}"
         C.dispose_quantized(b, Q)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("M,N,K,kernel", [(130, 392, 776, "codes mfma 128x64"), (70, 264, 1160, "codes mfma 128x64"),
+                                          (900, 2624, 328, "codes mfma 128x128"), (384, 8192, 256, "codes mfma 128x128")])
+def test_quantized_loader_geglu(b, M, N, K, kernel, bits, dtype):
+    """The 128-row kernel's dequantizing loader (its two register sets rotating
+    over an even and an odd number of K stages, K tails among them) with GeGLU
+    and a residual: the oracle's values (max-rel <= 1e-2), and the bits of the
+    rows in a call of the large-M kernel on the weight dequantized once."""
+    from laya_hip import compose as C
+    rng = np.random.default_rng(M + K + bits)
+    assert linear_kernel(b, M, N, K, True, bits) == kernel
+    h, q, sf, zf = _quantized(rng, 2 * N, K, bits, 8 if K % 64 else 64)
+    Q = C.upload_quantized(b, h, dtype)
+    x, r = rounded(rng.standard_normal((M, K)), dtype), rounded(rng.standard_normal((M, N)), dtype)
+
+    def run(rows):
+        X, R = (b.fromHost(to_host(np.resize(a, (rows, a.shape[1])), dtype)) for a in (x, r))
+        y = b.add(R, b.geglu(C.quantized_linear(b, X, Q)))
+        out, got = np.asarray(b.read(y).data), read32(b, y)
+        for t in (X, R, y):
+            b.dispose(t)
+        return out, got
+    small, got = run(M)
+    np.testing.assert_array_equal(small, run(large_m_rows(b, N, K, True))[0][:M])
+    rows = _rows(M, rng)
+    lin = rounded(cr.quantized_linear(x[rows], q, sf, zf, 8 if K % 64 else 64, dtype=dtype), dtype)
+    assert max_rel(got[rows], r[rows] + rounded(cr.geglu(lin), dtype)) <= 1e-2
+    C.dispose_quantized(b, Q)
 
 
 @pytest.mark.parametrize("bits,mode", [(8, "symmetric"), (4, "affine"), (8, "affine"), (4, "symmetric")])
@@ -338,15 +375,16 @@ def test_small_output_linear_epilogues(b):
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
-def test_small_m_slab_edges_and_bits_equal_large_m(b, dtype):
-    """The weight-stationary small-M kernel (16-bit weights, K % 64 == 0) on
-    its edges: rows not a multiple of 32, output widths that end inside a
-    32-column block, a bias that is an offset view (not 8-byte aligned),
-    GeGLU, residuals, K from 64 to 1152.  Against the oracle (max-rel 2e-3 /
-    8e-3), and bit for bit against the large-M kernel: the same X rows placed
-    in a 4096-row input give the same output rows.  (Output rows of a length
-    that is not a multiple of 8 take the f32 SIMT kernels instead, whose
-    summation order depends on the shape.)"""
+def test_small_m_edges_and_bits_equal_large_m(b, dtype):
+    """Calls of few rows (16-bit weights, K % 64 == 0) on their edges: rows not
+    a multiple of 32, output widths that end inside a 32-column block, a bias
+    that is an offset view (not 8-byte aligned), GeGLU, residuals, K from 64 to
+    1152.  Against the oracle (max-rel 2e-3 / 8e-3), and bit for bit against the
+    large-M kernel: the same X rows in a call that it takes give the same
+    output rows (96 x 64 weights, which it takes at no row count: another
+    tile of the ring).  (Output rows of a length that is not a multiple of 8
+    take the f32 SIMT kernels instead, whose summation order depends on the
+    shape.)"""
     rng = np.random.default_rng(21)
     cases = [(77, 784, 192, True, "offset", False), (300, 2304, 768, True, "aligned", False),
              (1, 768, 1152, False, "aligned", True), (129, 200, 1024, False, None, True),
@@ -369,10 +407,10 @@ def test_small_m_slab_edges_and_bits_equal_large_m(b, dtype):
         ref = r + ref if resid else ref
         err = max_rel(got, ref)
         assert err <= (2e-3 if dtype == "f16" else 8e-3), f"M={M} N={N2} K={K} geglu={geglu}: {err:.2e}"
-        # the same rows through the large-M kernel
-        xb = np.concatenate([x, rounded(rng.standard_normal((4096 - M, K)), dtype)])
-        rb = np.concatenate([r, rounded(rng.standard_normal((4096 - M, N)), dtype)])
-        XB, RB = b.fromHost(to_host(xb, dtype)), b.fromHost(to_host(rb, dtype))
+        # the same rows through another kernel
+        ML = 24576 if (N, K) == (96, 64) else large_m_rows(b, N, K, geglu)
+        assert linear_kernel(b, M, N, K, geglu) != linear_kernel(b, ML, N, K, geglu)
+        XB, RB = b.fromHost(to_host(np.resize(x, (ML, K)), dtype)), b.fromHost(to_host(np.resize(r, (ML, N)), dtype))
         yb = b.linear(XB, Wt, Bt)
         yb = b.geglu(yb) if geglu else yb
         yb = b.add(RB, yb) if resid else yb
@@ -383,13 +421,13 @@ def test_small_m_slab_edges_and_bits_equal_large_m(b, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
-def test_small_m_slab_takes_panel_operands(b, dtype):
-    """The small-M slab kernel reads x in panel order (HB_X_PANEL) and writes
-    a GeGLU output in panel order (HB_Y_PANEL), through the C ABI: bit for bit
+def test_small_m_takes_panel_operands(b, dtype):
+    """A call of few rows reads x in panel order (HB_X_PANEL) and writes a
+    GeGLU output in panel order (HB_Y_PANEL), through the C ABI: bit for bit
     the row-major results, for row counts that are not multiples of 32 (the
-    panel's padding rows) and a K longer than the registers (1152).  Calls
-    that take the 128 x 128 kernel, and small-M quantized calls, refuse
-    panel operands."""
+    panel's padding rows) and a K of 1152.  Calls past the bounds that
+    laya_hip.h gives, and quantized calls below M = 4096, refuse panel
+    operands."""
     from laya_hip import ffi as F
     rng = np.random.default_rng(31)
     dt = F.HB_F16 if dtype == "f16" else F.HB_BF16
@@ -402,7 +440,7 @@ def test_small_m_slab_takes_panel_operands(b, dtype):
     for (M, N2, K, geglu, with_bias) in [(1, 768, 768, False, False), (33, 2304, 768, True, True),
                                          (100, 768, 1152, False, True), (128, 2304, 768, False, False),
                                          (128, 2304, 768, True, False)]:
-        print(f"slab panel M={M} N={N2} K={K} geglu={geglu} {dtype}", flush=True)
+        print(f"small panel M={M} N={N2} K={K} geglu={geglu} {dtype}", flush=True)
         No = N2 // 2 if geglu else N2
         x = rounded(rng.standard_normal((M, K)), dtype)
         w = rounded(rng.normal(0, 0.05, (N2, K)), dtype)
@@ -429,7 +467,7 @@ def test_small_m_slab_takes_panel_operands(b, dtype):
             m.release()
         for t in (X, Wt, Bt):
             b.dispose(t)
-    # 2048 rows of a 2304-wide product take the 128 x 128 kernel: refused
+    # 2048 rows of a 2304-wide product are past the small calls' bound: refused
     x = b._malloc(2048 * 768 * 2)
     w = b._malloc(2304 * 768 * 2)
     y = b._malloc(2048 * 2304 * 2)  # sized for the call, which is refused before any launch

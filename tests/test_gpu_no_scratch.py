@@ -9,7 +9,7 @@ import contextlib
 import numpy as np
 import pytest
 
-from gpu_util import to_host
+from gpu_util import linear_kernel, to_host
 from laya_hip import ffi as F
 from laya_hip.host import HostTensor
 
@@ -68,9 +68,7 @@ def _qlinear(b, M, N, K, bits, dtype, geglu=False):
 @pytest.mark.parametrize("M,N,K,bits,geglu", [(33, 200, 768, 8, False), (130, 768, 1152, 4, False), (130, 264, 768, 4, True),
                                               (2100, 3072, 384, 8, False), (2100, 2304, 320, 4, False)])
 def test_quantized_linear_without_scratch(b, M, N, K, bits, geglu, dtype):
-    name = F.C.create_string_buffer(64)
-    b.n.call("kernel", "hb_linear_kernel", b.cus, K, M, N, K, bits, F.HB_EPI_GEGLU if geglu else 0, name, len(name))
-    assert not name.value.startswith(b"codes")  # with scratch: dequantized first
+    assert not linear_kernel(b, M, N, K, geglu, bits).startswith("codes")  # with scratch: dequantized first
     call, Y, n, _held = _qlinear(b, M, N, K, bits, dtype, geglu)
     call()
     want = _bits(b, Y, n)
