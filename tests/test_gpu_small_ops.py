@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from gpu_util import max_rel, read32, rounded, to_host
+from laya_hip.host import HostTensor
 from oracle import cpu_ref as cr
 
 pytestmark = pytest.mark.gpu
@@ -81,3 +82,17 @@ def test_dot_vectors(b, dtype, M, N, K):
             assert (np.abs(got - (x6 @ w6.T + bias)) <= bound).all()
         else:
             assert max_rel(got, cr.linear(x, w, bias)) <= {"f16": 2e-3, "bf16": 8e-3}[dtype]
+
+
+def test_bf16_stores_round_to_nearest_even(b):
+    """f32 -> bf16 over every upper half and the lower halves around the tie:
+    numpy's integer rounding bit for bit, subnormals and infinities included,
+    and a NaN (whatever its payload's upper bits) stays a NaN."""
+    hi = np.arange(65536, dtype=np.uint32) << 16
+    bits = (hi[:, None] | np.array([0, 1, 0x7fff, 0x8000, 0x8001, 0xffff], np.uint32)).reshape(-1)
+    got = np.asarray(b.read(b.cast(b.fromHost(HostTensor("f32", bits.shape, bits.view(np.float32))), "bf16")).data)
+    got = got.view(np.uint16)
+    nan = np.isnan(bits.view(np.float32))
+    want = ((bits.astype(np.uint64) + 0x7fff + ((bits >> 16) & 1)) >> 16).astype(np.uint16)
+    np.testing.assert_array_equal(got[~nan], want[~nan])
+    assert ((got[nan] & 0x7fff) > 0x7f80).all()
