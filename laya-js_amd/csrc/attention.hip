@@ -62,6 +62,7 @@ constexpr int kNW = kBQ / (16 * kQB);  // waves per block
 constexpr int kNT = kNW * 64;          // threads per block
 constexpr int kBK = 64;   // keys per tile
 constexpr int kMaxKeyTiles = 1024;  // Lk <= 65536 on the MFMA path
+constexpr int kRW = 4;    // sdpa32_ring: waves per block, 32 queries each
 
 // ------------------------------------------------------------------ mask summary
 
@@ -241,6 +242,30 @@ __device__ __forceinline__ void store_pair(uint4v lo, uint4v hi, bool rot, int c
   *(uint4v*)(lds + (KSWZ ? k_swz(row, c + 4) : qk_swz(row, c + 4))) = hi;
 }
 
+// Where a block works, of one per (b, h, query tile) on a 1-D grid.  Blocks are
+// dealt to the 8 XCDs in turn (block i on XCD i % 8).  The query tiles of one
+// (b, h) read the same K / V rows and mask bytes, so they are consecutive blocks
+// of one XCD's share and share its L2; the (b, h) pairs are dealt to the XCDs
+// in turn, which spreads sequences of different lengths (and work).  Without a
+// multiple of 8 pairs the blocks take (b, h, query tile) in order, or, with
+// RUNS, in contiguous runs per XCD.
+template <bool RUNS>
+__device__ __forceinline__ void sdpa_block(int nqt, int nh, int& qt, int& b, int& h) {
+  const int nbh = (int)(gridDim.x / nqt);
+  int bh;
+  if ((nbh & 7) == 0) {
+    const int x = blockIdx.x & 7, idx = blockIdx.x >> 3;
+    qt = idx % nqt;
+    bh = (idx / nqt) * 8 + x;
+  } else {
+    const uint32_t t = RUNS ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
+    qt = t % nqt;
+    bh = t / nqt;
+  }
+  h = bh % nh;
+  b = bh / nh;
+}
+
 template <bool BF16>
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void sdpa_mfma(const uint16_t* __restrict__ Q, S4 qs, const uint16_t* __restrict__ K,
                                                  S4 ks, const uint16_t* __restrict__ V, S4 vs,
@@ -256,24 +281,8 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void s
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, li = lane & 15;
-  // One block per (b, h, query tile) on a 1-D grid.  Blocks are dealt to the
-  // 8 XCDs in turn (block i on XCD i % 8).  The query tiles of one (b, h)
-  // read the same K / V rows and mask bytes, so they go to one XCD as
-  // consecutive blocks of its share (they run together and share its L2),
-  // and the (b, h) pairs are dealt to the XCDs in turn, which spreads
-  // sequences of different lengths (and work) evenly over them.  Without a
-  // multiple of 8 pairs the blocks take (b, h, query tile) in order.
-  const int nbh = (int)(gridDim.x / nqt);
-  int qt, bh;
-  if ((nbh & 7) == 0) {
-    const int x = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    qt = idx % nqt;
-    bh = (idx / nqt) * 8 + x;
-  } else {
-    qt = blockIdx.x % nqt;
-    bh = blockIdx.x / nqt;
-  }
-  const int h = bh % nh, b = bh / nh;
+  int qt, b, h;
+  sdpa_block<false>(nqt, nh, qt, b, h);
   const int nkt = (Lk + kBK - 1) / kBK;
   const int q0 = qt * kBQ;
   const uint16_t* Qb = Q + b * qs.s[0] + h * qs.s[1];
@@ -599,15 +608,6 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void s
 
 // ------------------------------------------------------------------ 32-query MFMA kernel
 
-// 16 bytes per lane from buffer `rs` at byte offset `voff` straight into LDS:
-// lane l fills [lds + 16 l, + 16); an offset past the buffer's records writes
-// zeros.  Inline asm, so that the compiler neither holds later LDS reads of the
-// other buffer behind it nor counts it in its own waits (an extra load in
-// flight only makes those stronger); the caller waits for it (vmcnt(0)).
-__device__ __forceinline__ void buffer_to_lds16(const uint4v& rs, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
-               : "memory", "m0");
-}
 typedef short short4t __attribute__((ext_vector_type(4)));
 // Transposing LDS read: within 16 lanes, lanes 4r .. 4r + 3 point at 4 x 4
 // consecutive values of row r; lane c gets column c's 4 rows.
@@ -842,40 +842,19 @@ __device__ __forceinline__ void wave32_store(const Wave32& w, uint16_t* O, const
     }
 }
 
-// Where a block works: the query tiles of one (b, h) read the same K / V rows,
-// so they are consecutive blocks of one XCD's share (blocks are dealt to the 8
-// XCDs in turn) and share its L2; the (b, h) pairs are dealt to the XCDs in
-// turn, which spreads sequences of different lengths, or, without a multiple
-// of 8 pairs, in contiguous runs.
-__device__ __forceinline__ void sdpa_block(int nqt, int nh, int& qt, int& b, int& h) {
-  const int nbh = (int)(gridDim.x / nqt);
-  int bh;
-  if ((nbh & 7) == 0) {
-    const int x = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    qt = idx % nqt;
-    bh = (idx / nqt) * 8 + x;
-  } else {
-    const int t = xcd_tile(blockIdx.x, gridDim.x);
-    qt = t % nqt;
-    bh = t / nqt;
-  }
-  h = bh % nh;
-  b = bh / nh;
-}
-
 // Classes of up to 64 key tiles: lane i gets the class of tile base + i for the
 // wave's own 32 queries qw .. (0 skip, 1 all visible, 2 mixed) in *mine;
-// returns the tiles some wave of the block (NW waves, queries q0 ..) needs.
-template <int NW>
-__device__ __forceinline__ uint64_t tile_classes(const uint8_t* cls, const uint8_t* mask, int b, int q0, int wave, int Lq,
-                                                 int Lk, int nkt, int base, int lane, uint32_t* mine) {
+// returns the tiles some wave of the block (queries q0 ..) needs.  cls: the
+// mask's summary, or null for no mask.
+__device__ __forceinline__ uint64_t tile_classes(const uint8_t* cls, int b, int q0, int wave, int Lq, int Lk, int nkt,
+                                                 int base, int lane, uint32_t* mine) {
   const int kt = base + lane, qw = q0 + 32 * wave;
   uint32_t any = 0, c = 0;
   if (kt < nkt) {
     if (cls != nullptr) {
       const int nqt128 = (Lq + kBQ - 1) / kBQ;
 #pragma unroll
-      for (int i = 0; i < NW; i++) {
+      for (int i = 0; i < kRW; i++) {
         const int qq = q0 + 32 * i;
         if (qq >= Lq) break;
         const uint32_t x =
@@ -886,7 +865,7 @@ __device__ __forceinline__ uint64_t tile_classes(const uint8_t* cls, const uint8
       const uint32_t c0 = c & 255u, c1 = qw + 16 < Lq ? c >> 8 : c0;  // (groups past Lq have class 0)
       c = c0 == c1 ? c0 : 2u;
     } else {
-      c = qw >= Lq ? 0u : mask == nullptr && (kt + 1) * kBK <= Lk ? 1u : 2u;
+      c = qw >= Lq ? 0u : (kt + 1) * kBK <= Lk ? 1u : 2u;
       any = 1;
     }
   }
@@ -896,7 +875,8 @@ __device__ __forceinline__ uint64_t tile_classes(const uint8_t* cls, const uint8
 
 // A K or V tile by direct-to-LDS loads: 8 pieces of 1 KB (8 rows); a piece's
 // lane l fills slot l % 8 of row l / 8, so it fetches chunk (l % 8) ^
-// kv_f(row).  Rows past Lk become zeros.
+// kv_f(row).  Rows past Lk become zeros (an offset past the buffer's records).
+// The caller waits for the loads (vmcnt(0)).
 __device__ __forceinline__ void dma_piece(const uint16_t* base, int64_t stride, int k0, int piece, int Lk, uint16_t* dst,
                                           int lane) {
   const uint64_t a = (uint64_t)(base + (int64_t)k0 * stride);
@@ -906,7 +886,7 @@ __device__ __forceinline__ void dma_piece(const uint16_t* base, int64_t stride, 
   const uint32_t off = __umul24(r, (uint32_t)stride) * 2u + (((lane & 7) ^ kv_f(r)) << 4);
   const uint32_t lds = (uint32_t)__builtin_amdgcn_readfirstlane(
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)(dst + piece * 512));
-  buffer_to_lds16(rs, k0 + r < Lk ? off : 0xfffffff0u, lds);
+  buffer_lds16(rs, k0 + r < Lk ? off : 0xfffffff0u, lds);
 }
 
 struct KPair {  // a K row's chunks c and c + 4 and their rotation
@@ -936,20 +916,20 @@ __device__ __forceinline__ void kpair_store(KPair& p, uint16_t* tile, int r, int
 // Three blocks per CU (168 VGPRs); four, at 128 VGPRs, measured the same, eight
 // waves a block slower (T 512 B 32 50 -> 58 us).  T = 2048, B = 16, 16 heads:
 // 566 -> 434 us (635 TFLOP/s), T = 8192, B = 1, 12 heads 460 -> 322 us.
-template <bool BF16, int NW, bool ROPEK>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(3))) void sdpa32_ring(
+template <bool BF16, bool ROPEK>
+__global__ __launch_bounds__(kRW * 64) __attribute__((amdgpu_waves_per_eu(3))) void sdpa32_ring(
     const uint16_t* __restrict__ Q, S4 qs, const uint16_t* __restrict__ K, S4 ks, const uint16_t* __restrict__ V, S4 vs,
     const uint8_t* __restrict__ mask, S4 ms, int mask_vec, const uint8_t* __restrict__ cls, uint16_t* __restrict__ O,
     S4 os, int Lq, int Lk, float scale_log2, const float2* __restrict__ tabq, const float2* __restrict__ tabk, int pK,
     int nqt, int nh) {
-  static_assert(NW == 4, "K staging: one chunk pair per thread");
+  static_assert(kRW == 4, "K staging: one chunk pair per thread");
   __shared__ __attribute__((aligned(16))) uint16_t Ks[2][kBK * 64];
   __shared__ __attribute__((aligned(16))) uint16_t Vs[2][kBK * 64];
   const int tid = threadIdx.x, lane = tid & 63, lg = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int qt, b, h;
-  sdpa_block(nqt, nh, qt, b, h);
-  const int q0 = qt * 32 * NW, q = q0 + 32 * wave + (lane & 31), qc = q < Lq ? q : Lq - 1;
+  sdpa_block<true>(nqt, nh, qt, b, h);
+  const int q0 = qt * 32 * kRW, q = q0 + 32 * wave + (lane & 31), qc = q < Lq ? q : Lq - 1;
   const int nkt = (Lk + kBK - 1) / kBK;
   const uint16_t* Kb = K + b * ks.s[0] + h * ks.s[1];
   const uint16_t* Vb = V + b * vs.s[0] + h * vs.s[1];
@@ -957,13 +937,13 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(3))) vo
 
   int base = 0;
   uint32_t mine;
-  uint64_t need = tile_classes<NW>(cls, mask, b, q0, wave, Lq, Lk, nkt, 0, lane, &mine);
+  uint64_t need = tile_classes(cls, b, q0, wave, Lq, Lk, nkt, 0, lane, &mine);
   // the next tile some wave needs (nkt: none) and its class for this wave
   auto next_tile = [&](uint32_t* c) -> int {
     while (need == 0) {
       base += 64;
       if (base >= nkt) return nkt;
-      need = tile_classes<NW>(cls, mask, b, q0, wave, Lq, Lk, nkt, base, lane, &mine);
+      need = tile_classes(cls, b, q0, wave, Lq, Lk, nkt, base, lane, &mine);
     }
     const int i = __builtin_ctzll(need);
     need &= need - 1;
@@ -978,12 +958,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(3))) vo
   auto fetch = [&](int kt, int bf) __attribute__((always_inline)) {
     const int k0 = kt * kBK;
 #pragma unroll
-    for (int i = 0; i < 8 / NW; i++) dma_piece(Vb, vs.s[2], k0, wave * (8 / NW) + i, Lk, Vs[bf], lane);
+    for (int i = 0; i < 8 / kRW; i++) dma_piece(Vb, vs.s[2], k0, wave * (8 / kRW) + i, Lk, Vs[bf], lane);
     if constexpr (ROPEK) {
       kpair_load(kp, Kb, ks.s[2], tabk, k0, kr, kc, Lk);
     } else {
 #pragma unroll
-      for (int i = 0; i < 8 / NW; i++) dma_piece(Kb, ks.s[2], k0, wave * (8 / NW) + i, Lk, Ks[bf], lane);
+      for (int i = 0; i < 8 / kRW; i++) dma_piece(Kb, ks.s[2], k0, wave * (8 / kRW) + i, Lk, Ks[bf], lane);
     }
   };
   // everything requested has landed (before the barrier that publishes it)
@@ -1487,8 +1467,8 @@ static void sdpa_impl(uintptr_t ctx, int dt, uintptr_t q, const int64_t* qs, uin
         tk = nullptr;
       }
       const int mask_vec = mask && ms[3] == 1 && mask % 16 == 0 && ms[0] % 16 == 0 && ms[2] % 16 == 0;
-      auto kern = dt == HB_F16 ? (tk ? sdpa32_ring<false, 4, true> : sdpa32_ring<false, 4, false>)
-                               : (tk ? sdpa32_ring<true, 4, true> : sdpa32_ring<true, 4, false>);
+      auto kern = dt == HB_F16 ? (tk ? sdpa32_ring<false, true> : sdpa32_ring<false, false>)
+                               : (tk ? sdpa32_ring<true, true> : sdpa32_ring<true, false>);
       kern<<<(unsigned)nblk, 256, 0, st>>>((const uint16_t*)q, Qs, (const uint16_t*)k, Ks, (const uint16_t*)v, Vs,
                                            (const uint8_t*)mask, Ms, mask_vec, info, (uint16_t*)o, Os, (int)Lq, (int)Lk,
                                            sl2, tq, tk, pK, nqt, (int)H);

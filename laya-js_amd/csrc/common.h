@@ -235,6 +235,21 @@ inline int64_t numel(const int64_t* shape, int rank) {
   return n;
 }
 
+// 16 bytes per lane from buffer resource `rs` at byte offset voff (+ soff) straight
+// into LDS: lane l fills [lds + 16 l, + 16), `lds` being wave-uniform; an offset
+// past the buffer's records writes zeros.  Inline asm, so that the compiler
+// neither holds LDS reads of other buffers behind it nor counts it in its own
+// waits (a load in flight only makes those stronger); the caller waits (vmcnt).
+__device__ __forceinline__ void buffer_lds16(const uint4v& rs, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
+               : "memory", "m0");
+}
+__device__ __forceinline__ void buffer_lds16(const uint4v& rs, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rs), "s"(soff),
+               "s"(lds)
+               : "memory", "m0");
+}
+
 inline unsigned grid_for(int64_t n, int block) {
   int64_t g = (n + block - 1) / block;
   if (g > (1 << 30)) g = 1 << 30;

@@ -407,8 +407,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_mfma(const uint16_t* __restr
 
 // ------------------------------------------------------------------ ring MFMA kernel
 
-// GEMM for 16-bit weights and K % 64 == 0, from one row up to where the large-M
-// kernel's tiles fill the chip.  Both operands go to an LDS ring of NST 64-wide K
+// GEMM for 16-bit weights and K % 64 == 0 in calls of few tiles (ring_tile says
+// how few).  Both operands go to an LDS ring of NST 64-wide K
 // stages by direct loads (no registers, so requests run stages ahead whatever the
 // wave is doing), with one barrier per stage; waves of 32 x 32 outputs (32 x 64 in
 // the widest tile) read each k16 step's fragments one step ahead.
@@ -424,14 +424,6 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_mfma(const uint16_t* __restr
 // Same MFMA, operand order (W rows as the A operand, X rows as the B operand) and
 // ascending k16 steps as the other kernels: a row's bits do not depend on M or on
 // the tile.
-// 16 bytes per lane from buffer `rs` at byte offsets voff + soff straight into
-// LDS [lds + 16 lane, + 16).  Inline asm: the compiler neither holds LDS reads
-// behind it nor counts it in its waits; the caller waits (vmcnt).
-__device__ __forceinline__ void ring_dma16(const uint4v& rs, uint32_t voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rs), "s"(soff),
-               "s"(lds)
-               : "memory", "m0");
-}
 template <int N>
 __device__ __forceinline__ void ring_wait_barrier() {
   // this wave's loads up to the stage about to be read have landed, its LDS
@@ -515,7 +507,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_ring(const uint16_t* __restr
   auto issue = [&](int kt, int slot, int i0, int i1) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = i0; i < i1; i++)
-      ring_dma16(rsrc[i], off[i], (uint32_t)kt * step[i], lds0 + (uint32_t)(slot * STAGE * 2 + (wave * PW + i) * 1024));
+      buffer_lds16(rsrc[i], off[i], (uint32_t)kt * step[i], lds0 + (uint32_t)(slot * STAGE * 2 + (wave * PW + i) * 1024));
   };
 
   float16v acc[TM][TN];
@@ -1535,8 +1527,9 @@ inline bool ring_beats_arow(int64_t M, int64_t N_out, int64_t K, bool geglu, int
   return ring < arow;
 }
 
-// Calls below M = 4096 that take panel-order operands (laya_hip.h): 16-bit
-// weights, and few enough rows that the producer's panel costs nothing.
+// Calls below M = 4096 that take panel-order operands: 16-bit weights within the
+// bounds that laya_hip.h gives its callers.  They are the interface's and not
+// gemm_ring's, which takes panel order at any size with K % 64 == 0.
 inline bool small_panel_path(int64_t M, int64_t N_out, int64_t K, bool geglu, int cus) {
   const int64_t tiles_n = (N_out + 31) / 32, chunks = (M + 127) / 128;
   return K % 64 == 0 && K * 32 * (geglu ? 2 : 1) * 2 <= 160 * 1024 && tiles_n * chunks <= cus;
