@@ -1495,8 +1495,9 @@ inline const char* linear_kernel_name(LinearKernel k) {
 //   the 128-row kernel 20.5; 3072 x 2304 x 768 (216) 20.4, 22.5; with weights
 //   from HBM 23.1 / 20.6 and 23.7 / 23.5;
 // - 64 x 64 with three stages in up to three rounds where the 128-row kernel's
-//   128 x 128 tiles begin a second round (two fit a CU): 4095 x 2304 x 768 30 /
-//   36, 3072 x 3072 x 1024 38 / 44;
+//   128 x 128 tiles begin a second round (two fit a CU), unless the weight is
+//   the wider side: 4095 x 2304 x 768 30 / 36, 3072 x 3072 x 1024 38 / 44, 1792 x
+//   5248 x 1024 46 / 44;
 // - else none below M = 4096 (`wide` false): the 128-row kernel reads half as
 //   much LDS per product as a 64 x 64 tile.  1536 x 2304 x 768 18.0 / 16.0 us,
 //   2048 x 2624 x 1024 GeGLU 56.8 / 43.4, 3840 x 4096 x 1024 68.1 / 51.9.
@@ -1508,7 +1509,8 @@ inline bool ring_tile(int cus, int64_t M, int64_t wrows, int64_t K, bool geglu, 
   else if (tiles(128, 64) <= cus) *tile = LinearKernel::kRing128x64;
   else if (t64 <= 3 * (int64_t)cus) *tile = LinearKernel::kRing64x64x3;
   else if (t256 > cus / 2 && t256 <= cus && !geglu && K >= 512 && K <= 1536) *tile = LinearKernel::kRing128x256;
-  else if (wide || (t64 <= 9 * (int64_t)cus && tiles(128, 128) > 2 * (int64_t)cus)) *tile = LinearKernel::kRing64x64x3;
+  else if (wide || (t64 <= 9 * (int64_t)cus && tiles(128, 128) > 2 * (int64_t)cus && M >= wrows))
+    *tile = LinearKernel::kRing64x64x3;
   else return false;
   return true;
 }

@@ -27,6 +27,7 @@ def kernel(M, N, K, flags=0, ldx=None, cus=256, bits=0):
     (3840, 1024, 4096, 0, "mfma 128x64"), (700, 50368, 768, 0, "mfma 128x128"),
     # its 128 x 128 tiles just over two a CU: the ring's three rounds
     (3840, 2304, 768, 0, "ring 64x64 three"), (3072, 3072, 1024, 0, "ring 64x64 three"),
+    (1792, 5248, 1024, 0, "mfma 128x128"),
     # other K; from M = 4096
     (512, 768, 776, 0, "mfma 128x64"), (4096, 2304, 768, 0, "arow 192"), (4096, 768, 768, 0, "ring 64x64 three"),
     (16384, 1024, 1024, 0, "arow 128"), (4096, 768, 776, 0, "arow 192 tail"),
