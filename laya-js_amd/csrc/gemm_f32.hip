@@ -264,7 +264,9 @@ static void launch_f32(hipStream_t st, int cus, const float* x, int64_t ldx, con
                        const float* r, int64_t ldr, float* y, int64_t ldy, int M, int N, int K) {
   const int64_t wrows = GEGLU ? 2 * (int64_t)N : N;
   // By the number of 32 x 32 tiles, and not by GEGLU: the fused and the
-  // separate GeGLU take the same sums.  Both sides of each line, us at K = 768
+  // separate GeGLU take the same sums.  The tiles split K eight, four and two
+  // ways, so (unlike a 16-bit row's) an f32 row's last bits depend on the call's
+  // row count.  Both sides of each line, us at K = 768
   // (small / middle / large):
   // - up to two tiles per CU: 93 x 2304 (216 tiles) 7.8 / 11.7 / 19, 512 x 768
   //   (384) 11.6 / 11.6 / 18.8, 256 x 2304 (576) 17.4 / 19.4 / 19.7, and with
