@@ -321,7 +321,7 @@ extern "C" int hb_linear_kernel(int cus, int64_t ldx, int64_t M, int64_t N, int6
   const int64_t ld = (flags & HB_X_PANEL) ? K : ldx;
   const bool codes = bits != 0 && !dequantizes_first(cus, M, N, K, ld, geglu);
   const LinearKernel k = codes ? code_kernel(cus, M, N, geglu)
-                               : linear_kernel(cus, M, N, K, ld, geglu, flags & (HB_X_PANEL | HB_Y_PANEL));
+                               : linear_kernel(cus, M, N, K, ld, geglu, flags & (HB_X_PANEL | HB_Y_PANEL), bits != 0);
   std::snprintf(name, cap, "%s%s", codes ? "codes " : "", linear_kernel_name(k));
   HB_API_END
 }
@@ -434,8 +434,7 @@ extern "C" int hb_qlinear(uintptr_t ctx, int dt, uintptr_t x, int64_t ldx, uintp
       else if (mode == 0) launch_dequant_rows<4, false>(st, cus, dt, q, wd, rows, k);
       else launch_dequant_rows<4, true>(st, cus, dt, q, wd, rows, k);
       check_launch("hb_qlinear (dequantize)");
-      QW none{nullptr, nullptr, nullptr, 0, 1};
-      mfma_dtype<0, false, false>(dt, geglu, st, cus, pan, X, ldx, wd, none, Bp, Rp, ldr, Yp, ldy, m, n, k);
+      mfma_dtype<0, false, false>(dt, geglu, st, cus, pan, X, ldx, wd, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
     } else if (bits == 8 && mode == 0) mfma_dtype<8, false, false>(dt, geglu, st, cus, pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
     else if (bits == 8) mfma_dtype<8, true, false>(dt, geglu, st, cus, pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);
     else if (mode == 0) mfma_dtype<4, false, false>(dt, geglu, st, cus, pan, X, ldx, nullptr, q, Bp, Rp, ldr, Yp, ldy, m, n, k);

@@ -1488,12 +1488,15 @@ inline const char* linear_kernel_name(LinearKernel k) {
 //   768 x 2304 x 768 (216) 8.7 / 8.4 / 9.3 (12.3);
 // - 64 x 64 with three stages while three fit a CU: 1024 x 3072 x 768 15.4 /
 //   15.7 / 12.6 (16.4), 4096 x 768 x 768 12.1 / 14.0 / 11.1;
-// - 128 x 256, one round of them that fills more than half the CUs, K of 512 to
-//   1536 (beyond that its three stages wait for weights from HBM: 2048 x 2304 x
-//   3072 69 against 58 us) and no GeGLU (whose epilogue costs its single block a
-//   CU more: 2048 x 1152 x 768 21.5 / 19.7): 2048 x 2304 x 768 (144 tiles) 18.3,
-//   the 128-row kernel 20.5; 3072 x 2304 x 768 (216) 20.4, 22.5; with weights
-//   from HBM 23.1 / 20.6 and 23.7 / 23.5;
+// - 128 x 256, one round of them that fills three quarters of the CUs (half, if
+//   the weight was just written: `cached`), K of 512 to 1536 (beyond that
+//   its three stages wait for weights from HBM: 2048 x 2304 x 3072 69 against 58
+//   us) and no GeGLU (whose epilogue costs its single block a CU more: 2048 x 1152
+//   x 768 21.5 / 19.7).  Against the 128-row kernel, weights in the caches / from
+//   HBM: 2048 x 2304 x 768 (144 tiles) 18.3 and 20.5 / 23.1 and 20.6, 2048 x 3072 x
+//   768 (192) 20.9 and 22.4 / 23.8 and 23.1, 3072 x 2304 x 768 (216) 20.4 and 22.5 /
+//   23.7 and 23.5; a 2048-token f16 forward takes 1.98 ms without it, 2.05 with,
+//   a q4 one, whose weights are copies just dequantized, 2.19 and 2.17;
 // - 64 x 64 with three stages in up to three rounds where the 128-row kernel's
 //   128 x 128 tiles begin a second round (two fit a CU), unless the weight is
 //   the wider side: 4095 x 2304 x 768 30 / 36, 3072 x 3072 x 1024 38 / 44, 1792 x
@@ -1501,14 +1504,16 @@ inline const char* linear_kernel_name(LinearKernel k) {
 // - else none below M = 4096 (`wide` false): the 128-row kernel reads half as
 //   much LDS per product as a 64 x 64 tile.  1536 x 2304 x 768 18.0 / 16.0 us,
 //   2048 x 2624 x 1024 GeGLU 56.8 / 43.4, 3840 x 4096 x 1024 68.1 / 51.9.
-inline bool ring_tile(int cus, int64_t M, int64_t wrows, int64_t K, bool geglu, bool wide, LinearKernel* tile) {
+inline bool ring_tile(int cus, int64_t M, int64_t wrows, int64_t K, bool geglu, bool wide, bool cached,
+                      LinearKernel* tile) {
   auto tiles = [&](int bm, int bn) { return ((M + (int64_t)bm - 1) / bm) * ((wrows + bn - 1) / bn); };
   const int64_t t64 = tiles(64, 64), t256 = tiles(128, 256);
   if (tiles(32, 64) <= cus) *tile = LinearKernel::kRing32x64;
   else if (t64 <= cus) *tile = K < 2048 ? LinearKernel::kRing64x64 : LinearKernel::kRing64x64k;
   else if (tiles(128, 64) <= cus) *tile = LinearKernel::kRing128x64;
   else if (t64 <= 3 * (int64_t)cus) *tile = LinearKernel::kRing64x64x3;
-  else if (t256 > cus / 2 && t256 <= cus && !geglu && K >= 512 && K <= 1536) *tile = LinearKernel::kRing128x256;
+  else if (t256 > (cached ? cus / 2 : cus * 3 / 4 - 1) && t256 <= cus && !geglu && K >= 512 && K <= 1536)
+    *tile = LinearKernel::kRing128x256;
   else if (wide || (t64 <= 9 * (int64_t)cus && tiles(128, 128) > 2 * (int64_t)cus && M >= wrows))
     *tile = LinearKernel::kRing64x64x3;
   else return false;
@@ -1560,16 +1565,17 @@ inline LinearKernel code_kernel(int cus, int64_t M, int64_t N_out, bool geglu) {
 
 // The kernel a call with 16-bit weights takes.  `ldx`: X's row stride, K in
 // panel order; `panel`: X or Y in panel order, which the 128-row kernel does
-// not take.  Every output keeps its MFMA sequence and epilogue, so the bits do
+// not take; `cached`: the weight is a copy that a kernel just wrote.  Every output keeps its MFMA sequence and epilogue, so the bits do
 // not depend on the choice.
-inline LinearKernel linear_kernel(int cus, int64_t M, int64_t N_out, int64_t K, int64_t ldx, bool geglu, bool panel) {
+inline LinearKernel linear_kernel(int cus, int64_t M, int64_t N_out, int64_t K, int64_t ldx, bool geglu, bool panel,
+                                  bool cached) {
   // 128-column tiles of the large-M kernel where N is a multiple of 128 and
   // not of 192 (N = 1024: 8 whole tiles instead of 5 1/3 of 192 columns)
   const bool n128 = !geglu && N_out % 192 != 0 && N_out % 128 == 0;
   const bool ring = ring_ok(ldx, K), large = arow_path(M);
   LinearKernel tile;
   if (ring && (!large || ring_beats_arow(M, N_out, K, geglu, n128 ? 128 : 192, cus)) &&
-      ring_tile(cus, M, geglu ? 2 * N_out : N_out, K, geglu, large || panel, &tile))
+      ring_tile(cus, M, geglu ? 2 * N_out : N_out, K, geglu, large || panel, cached, &tile))
     return tile;
   if (large || panel) {
     // (X rows too far apart for 32-bit offsets: the tail variant's are 64-bit)
@@ -1593,7 +1599,7 @@ inline LinearKernel linear_kernel(int cus, int64_t M, int64_t N_out, int64_t K, 
 // x 768 23.9 / 27.8).
 inline bool dequantizes_first(int cus, int64_t M, int64_t N_out, int64_t K, int64_t ldx, bool geglu) {
   if (arow_path(M) || (M >= 1024 && !thin_tiles(M, N_out, geglu, cus))) return true;
-  return is_ring(linear_kernel(cus, M, N_out, K, ldx, geglu, false)) &&
+  return is_ring(linear_kernel(cus, M, N_out, K, ldx, geglu, false, true)) &&
          (geglu ? 2 : 1) * N_out * K <= (K / 64 - 4) * 500000;
 }
 
@@ -1602,9 +1608,9 @@ void mfma_dispatch(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int
                           QW qw, const uint16_t* bias, const uint16_t* r, int64_t ldr, uint16_t* y, int64_t ldy, int M,
                           int N, int K) {
   // (codes are read by the 128-row kernel alone: hb_qlinear dequantizes them
-  // beforehand for the others)
+  // beforehand for the others, and passes them along with the copy)
   HB_REQUIRE(QB == 0 || !arow_path(M), "hb_qlinear: large-M quantized weights are dequantized before the GEMM");
-  const LinearKernel kern = QB == 0 ? linear_kernel(cus, M, N, K, (pan & HB_X_PANEL) ? K : ldx, GEGLU, pan != 0)
+  const LinearKernel kern = QB == 0 ? linear_kernel(cus, M, N, K, (pan & HB_X_PANEL) ? K : ldx, GEGLU, pan != 0, qw.q != nullptr)
                                     : code_kernel(cus, M, N, GEGLU);
   if constexpr (QB == 0) {
     auto args = [&](auto launch) { launch(st, pan, x, ldx, w, bias, r, ldr, y, ldy, M, N, K); };

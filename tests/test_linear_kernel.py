@@ -19,7 +19,7 @@ def kernel(M, N, K, flags=0, ldx=None, cus=256, bits=0):
     (1, 768, 768, 0, "ring 32x64"), (93, 2304, 768, 0, "ring 32x64"), (256, 2304, 768, 0, "ring 64x64"),
     (768, 768, 3072, 0, "ring 64x64 long"), (512, 3072, 768, 0, "ring 128x64"), (512, 1152, 768, 1, "ring 128x64"),
     (1024, 2304, 768, 0, "ring 64x64 three"), (3840, 768, 768, 0, "ring 64x64 three"),
-    (2048, 2304, 768, 0, "ring 128x256"), (3584, 2304, 768, 0, "ring 128x256"), (2560, 3072, 1024, 0, "ring 128x256"),
+    (2048, 2304, 768, 0, "mfma 128x64"), (2048, 3072, 768, 0, "ring 128x256"), (3584, 2304, 768, 0, "ring 128x256"), (2560, 3072, 1024, 0, "ring 128x256"),
     # the 128-row kernel where the ring's tiles were slower: GeGLU, K = 3072, more than a round
     (2048, 1152, 768, 1, "mfma 128x64"), (3072, 1152, 768, 1, "mfma 128x128"), (2048, 2304, 3072, 0, "mfma 128x64"),
     (700, 2624, 1024, 1, "mfma 128x64"), (2048, 2624, 1024, 1, "mfma 128x128"), (3072, 2624, 1024, 1, "mfma 128x128"),
@@ -57,7 +57,7 @@ def test_panel_order_operands_never_meet_the_kernel_without_them():
 @pytest.mark.parametrize("M,N,K,geglu,want", [
     (1, 768, 768, 0, "ring 32x64"), (128, 2304, 768, 0, "ring 32x64"), (512, 768, 1152, 0, "ring 32x64"),
     (512, 1152, 768, 1, "ring 128x64"), (256, 2624, 1024, 1, "ring 128x64"), (1024, 3072, 1024, 0, "ring 64x64 three"),
-    (3072, 2304, 768, 0, "ring 128x256"), (3072, 2624, 1024, 1, "mfma 128x128"), (16384, 2304, 768, 0, "arow 192"),
+    (2048, 2304, 768, 0, "ring 128x256"), (3072, 2304, 768, 0, "ring 128x256"), (3072, 2624, 1024, 1, "mfma 128x128"), (16384, 2304, 768, 0, "arow 192"),
     # a short K chain, or a weight that is wide against it: the loader was faster
     (1, 48, 64, 0, "codes mfma 128x64"), (4000, 48, 64, 0, "codes mfma 128x64"), (256, 16384, 768, 0, "codes mfma 128x64"),
     (1, 50368, 768, 0, "codes mfma 128x128"), (33, 256000, 1024, 0, "codes mfma 128x128"),
