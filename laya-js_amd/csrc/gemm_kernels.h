@@ -1488,20 +1488,23 @@ inline const char* linear_kernel_name(LinearKernel k) {
 //   768 x 2304 x 768 (216) 8.7 / 8.4 / 9.3 (12.3);
 // - 64 x 64 with three stages while three fit a CU: 1024 x 3072 x 768 15.4 /
 //   15.7 / 12.6 (16.4), 4096 x 768 x 768 12.1 / 14.0 / 11.1;
-// - 128 x 256, one round of them that fills three quarters of the CUs (half, if
-//   the weight was just written: `cached`), K of 512 to 1536 (beyond that
-//   its three stages wait for weights from HBM: 2048 x 2304 x 3072 69 against 58
-//   us) and no GeGLU (whose epilogue costs its single block a CU more: 2048 x 1152
-//   x 768 21.5 / 19.7).  Against the 128-row kernel, weights in the caches / from
-//   HBM: 2048 x 2304 x 768 (144 tiles) 18.3 and 20.5 / 23.1 and 20.6, 2048 x 3072 x
-//   768 (192) 20.9 and 22.4 / 23.8 and 23.1, 3072 x 2304 x 768 (216) 20.4 and 22.5 /
-//   23.7 and 23.5; a 2048-token f16 forward takes 1.98 ms without it, 2.05 with,
-//   a q4 one, whose weights are copies just dequantized, 2.19 and 2.17;
+// - 128 x 256, one round of them: where the 128-row kernel does not take the call
+//   (`wide`) if it fills half the CUs: 4200 x 1536 x 384 14.3, 64 x 64 with three
+//   stages 16.5, 5500 x 768 x 3072 52.2 / 57.6.  Against the 128-row kernel from
+//   three quarters of the CUs on, or half for a weight just written (`cached`),
+//   for K of 512 to 1536 (beyond that the three stages wait for weights from HBM:
+//   2048 x 2304 x 3072 69 against 58 us) and without GeGLU (whose epilogue costs
+//   the single block of a CU more: 2048 x 1152 x 768 21.5 / 19.7); weights in the
+//   caches / from HBM: 2048 x 2304 x 768 (144 tiles) 18.3 and 20.5 / 23.1 and 20.6,
+//   2048 x 3072 x 768 (192) 20.9 and 22.4 / 23.8 and 23.1, 3072 x 2304 x 768 (216)
+//   20.4 and 22.5 / 23.7 and 23.5; a 2048-token f16 forward takes 1.98 ms without
+//   them at 144 tiles, 2.05 with, a q4 one, whose weights are copies just
+//   dequantized, 2.19 and 2.17;
 // - 64 x 64 with three stages in up to three rounds where the 128-row kernel's
 //   128 x 128 tiles begin a second round (two fit a CU), unless the weight is
 //   the wider side: 4095 x 2304 x 768 30 / 36, 3072 x 3072 x 1024 38 / 44, 1792 x
 //   5248 x 1024 46 / 44;
-// - else none below M = 4096 (`wide` false): the 128-row kernel reads half as
+// - else none below M = 4096 (not `wide`): the 128-row kernel reads half as
 //   much LDS per product as a 64 x 64 tile.  1536 x 2304 x 768 18.0 / 16.0 us,
 //   2048 x 2624 x 1024 GeGLU 56.8 / 43.4, 3840 x 4096 x 1024 68.1 / 51.9.
 inline bool ring_tile(int cus, int64_t M, int64_t wrows, int64_t K, bool geglu, bool wide, bool cached,
@@ -1512,7 +1515,8 @@ inline bool ring_tile(int cus, int64_t M, int64_t wrows, int64_t K, bool geglu, 
   else if (t64 <= cus) *tile = K < 2048 ? LinearKernel::kRing64x64 : LinearKernel::kRing64x64k;
   else if (tiles(128, 64) <= cus) *tile = LinearKernel::kRing128x64;
   else if (t64 <= 3 * (int64_t)cus) *tile = LinearKernel::kRing64x64x3;
-  else if (t256 > (cached ? cus / 2 : cus * 3 / 4 - 1) && t256 <= cus && !geglu && K >= 512 && K <= 1536)
+  else if (t256 > (cached || wide ? cus / 2 : cus * 3 / 4 - 1) && t256 <= cus &&
+           (wide || (!geglu && K >= 512 && K <= 1536)))
     *tile = LinearKernel::kRing128x256;
   else if (wide || (t64 <= 9 * (int64_t)cus && tiles(128, 128) > 2 * (int64_t)cus && M >= wrows))
     *tile = LinearKernel::kRing64x64x3;
@@ -1621,9 +1625,7 @@ void mfma_dispatch(hipStream_t st, int cus, unsigned pan, const uint16_t* x, int
       case LinearKernel::kRing64x64k: return args(launch_ring_t<64, 64, 2, 2, 5, BF16, GEGLU>);
       case LinearKernel::kRing64x64x3: return args(launch_ring_t<64, 64, 2, 2, 3, BF16, GEGLU>);
       case LinearKernel::kRing128x64: return args(launch_ring_t<128, 64, 4, 2, 4, BF16, GEGLU>);
-      case LinearKernel::kRing128x256:
-        if constexpr (!GEGLU) return args(launch_ring_t<128, 256, 4, 4, 3, BF16, GEGLU>);
-        break;
+      case LinearKernel::kRing128x256: return args(launch_ring_t<128, 256, 4, 4, 3, BF16, GEGLU>);
       case LinearKernel::kArow192: return arow(launch_arow<192, BF16, GEGLU, false>);
       case LinearKernel::kArow192Tail: return arow(launch_arow<192, BF16, GEGLU, true>);
       case LinearKernel::kArow128:

@@ -24,7 +24,8 @@ SHAPES = [(1, 8, 64, "ring 32x64"), (65, 72, 128, "ring 32x64"), (130, 200, 768,
           (2100, 2120, 128, "mfma 128x128")]
 GEGLU_SHAPES = [(1, 8, 64, "ring 32x64"), (65, 40, 128, "ring 32x64"), (300, 648, 2112, "ring 32x64"),
                 (520, 520, 192, "ring 64x64"), (520, 520, 2112, "ring 64x64 long"), (900, 648, 192, "ring 128x64"),
-                (1030, 1304, 64, "ring 64x64 three"), (1030, 1504, 64, "mfma 128x64"), (2100, 1064, 128, "mfma 128x128")]
+                (1030, 1304, 64, "ring 64x64 three"), (1030, 1504, 64, "mfma 128x64"), (2100, 1064, 128, "mfma 128x128"),
+                (4200, 520, 128, "ring 128x256")]
 
 
 @pytest.fixture(scope="module")

@@ -31,6 +31,7 @@ def kernel(M, N, K, flags=0, ldx=None, cus=256, bits=0):
     # other K; from M = 4096
     (512, 768, 776, 0, "mfma 128x64"), (4096, 2304, 768, 0, "arow 192"), (4096, 768, 768, 0, "ring 64x64 three"),
     (16384, 1024, 1024, 0, "arow 128"), (4096, 768, 776, 0, "arow 192 tail"),
+    (4200, 1536, 384, 0, "ring 128x256"), (4200, 640, 768, 1, "ring 128x256"), (5500, 768, 3072, 0, "ring 128x256"),
 ])
 def test_the_rule(M, N, K, geglu, want):
     assert kernel(M, N, K, GEGLU if geglu else 0) == want
